@@ -312,6 +312,20 @@ int saga_gemv(const saga_tensor* x, const saga_tensor* w, const saga_tensor* bia
               int32_t epilogue, saga_tensor* y, void* workspace, size_t workspace_bytes,
               saga_stream_t stream);
 
+/* The inverse of the packed layouts, for a prompt's GEMMs: n (1 to
+ * SAGA_UNPACK_MAX) packed weights (as saga_gemv takes them, K % 64 == 0 for
+ * 8-row tiles) to row-major out [N, K] (16-byte aligned rows) in one launch.
+ * head_rows > 0: the first rot_heads heads of head_rows (even, dividing N)
+ * packed rows go from rotary-pair order [0, d/2, 1, d/2 + 1, ...] to natural
+ * order (q/k heads of saga_gemv_rope_kv; one head of N rows undoes the
+ * gate/up interleave of SAGA_GEMV_SILU_PAIRS); head_rows 0 keeps the order. */
+#define SAGA_UNPACK_MAX 8
+typedef struct saga_unpack_item {
+  saga_tensor w, out;
+  int64_t rot_heads, head_rows;
+} saga_unpack_item;
+int saga_unpack_gemv(const saga_unpack_item* items, int32_t n, saga_stream_t stream);
+
 /* saga_gemv (STORE, bias, fused RMSNorm) of the fused q/k/v projection with
  * saga_rope_kv_append applied in its epilogue: one launch per layer for
  * projection + RoPE + cache append.  x [M, K] (M <= 32 new tokens), w bf16

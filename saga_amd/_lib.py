@@ -39,6 +39,10 @@ class SagaTensor(ctypes.Structure):
     ]
 
 
+class UnpackItem(ctypes.Structure):
+    _fields_ = [("w", SagaTensor), ("out", SagaTensor), ("rot_heads", ctypes.c_int64), ("head_rows", ctypes.c_int64)]
+
+
 class AtopnLayout(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int64) for n in (
         "scores", "scores_ld", "part_max", "part_sum", "part_tail", "nparts", "thresh",
@@ -75,6 +79,7 @@ _SIGS = {
     "saga_silu_mul": (ctypes.c_int, [_T, _T, _P]),
     "saga_gemv_workspace_bytes": (ctypes.c_size_t, [_I64, _I64, _I64]),
     "saga_gemv": (ctypes.c_int, [_T, _T, _T, ctypes.c_float, ctypes.c_int32, _T, _P, ctypes.c_size_t, _P]),
+    "saga_unpack_gemv": (ctypes.c_int, [ctypes.POINTER(UnpackItem), ctypes.c_int32, _P]),
     "saga_gemv_rope_kv": (ctypes.c_int, [_T, _T, _T, ctypes.c_float, _I64, _I64, _I64, ctypes.c_float, _P, _P,
                                          _T, _T, _T, _P, _P]),
     "saga_rope_table": (ctypes.c_int, [_P, _I64, _I64, ctypes.c_float, _P, _P]),
@@ -125,10 +130,8 @@ def dtype_code(dt: torch.dtype) -> int:
         raise TypeError(f"saga_amd: unsupported dtype {dt}") from None
 
 
-def tensor(t: torch.Tensor | None):
-    """saga_tensor descriptor of a torch tensor (None -> NULL)."""
-    if t is None:
-        return None
+def descriptor(t: torch.Tensor) -> SagaTensor:
+    """saga_tensor descriptor of a torch tensor."""
     if t.dim() > 4:
         raise ValueError("saga_amd: at most 4 dims")
     d = SagaTensor()
@@ -140,7 +143,12 @@ def tensor(t: torch.Tensor | None):
     for i in range(d.ndim):
         d.shape[i] = shape[i]
         d.stride[i] = stride[i]
-    return ctypes.byref(d)
+    return d
+
+
+def tensor(t: torch.Tensor | None):
+    """Reference to the saga_tensor descriptor of a torch tensor (None -> NULL)."""
+    return None if t is None else ctypes.byref(descriptor(t))
 
 
 def ptr(t: torch.Tensor | None):

@@ -732,6 +732,22 @@ int make_rope(int64_t N, int32_t dt, int64_t n_q, int64_t n_k, int64_t n_v, floa
   return SAGA_OK;
 }
 
+// A packed weight of K columns: contiguous [N/16, K/32, 16, 32] or, in 8-row
+// tiles, [N/8, K/64, 512] (the stride of a size-1 dim is immaterial).
+int check_packed(const saga_tensor* w, int64_t K) {
+  if (w->ndim == 4) {
+    if (w->shape[2] != 16 || w->shape[3] != 32 || w->shape[1] * 32 != K || w->stride[3] != 1 || w->stride[2] != 32 ||
+        (w->shape[1] > 1 && w->stride[1] != 512) || (w->shape[0] > 1 && w->stride[0] != w->shape[1] * 512))
+      return fail(SAGA_ERR_INVALID, "gemv: packed w must be contiguous [N/16, K/32, 16, 32] with K = x.shape[1]");
+  } else {
+    if (w->shape[2] != 512 || w->shape[1] * 64 != K || w->stride[2] != 1 ||
+        (w->shape[1] > 1 && w->stride[1] != 512) || (w->shape[0] > 1 && w->stride[0] != w->shape[1] * 512))
+      return fail(SAGA_ERR_INVALID, "gemv: 8-row packed w must be contiguous [N/8, K/64, 512] with K = x.shape[1]");
+  }
+  if (reinterpret_cast<uintptr_t>(w->data) % 16) return fail(SAGA_ERR_INVALID, "gemv: packed w must be 16-byte aligned");
+  return SAGA_OK;
+}
+
 // Validates x [M, K] and w [N, K] (bf16, 16-byte aligned rows) and an optional
 // bias [N] of a skinny GEMM and fills the shared fields of p.
 int make_gemv(const saga_tensor* x, const saga_tensor* w, const saga_tensor* bias, float rms_eps, GemvParams& p) {
@@ -743,19 +759,9 @@ int make_gemv(const saga_tensor* x, const saga_tensor* w, const saga_tensor* bia
   if (x->dtype != SAGA_DTYPE_BF16 || w->dtype != SAGA_DTYPE_BF16) return fail(SAGA_ERR_UNSUPPORTED, "gemv: bf16 only");
   const int64_t M = x->shape[0], K = x->shape[1];
   const int64_t N = packed ? w->shape[0] * 16 : packed8 ? w->shape[0] * 8 : w->shape[0];
-  if (packed) {
-    // [N/16][K/32][16][32], contiguous (the stride of a size-1 dim is immaterial)
-    if (w->shape[2] != 16 || w->shape[3] != 32 || w->shape[1] * 32 != K || w->stride[3] != 1 || w->stride[2] != 32 ||
-        (w->shape[1] > 1 && w->stride[1] != 512) || (w->shape[0] > 1 && w->stride[0] != w->shape[1] * 512))
-      return fail(SAGA_ERR_INVALID, "gemv: packed w must be contiguous [N/16, K/32, 16, 32] with K = x.shape[1]");
-    if (reinterpret_cast<uintptr_t>(w->data) % 16) return fail(SAGA_ERR_INVALID, "gemv: packed w must be 16-byte aligned");
-  } else if (packed8) {
-    // [N/8][K/64][512], contiguous
-    if (w->shape[2] != 512 || w->shape[1] * 64 != K || w->stride[2] != 1 ||
-        (w->shape[1] > 1 && w->stride[1] != 512) || (w->shape[0] > 1 && w->stride[0] != w->shape[1] * 512))
-      return fail(SAGA_ERR_INVALID, "gemv: 8-row packed w must be contiguous [N/8, K/64, 512] with K = x.shape[1]");
-    if (reinterpret_cast<uintptr_t>(w->data) % 16) return fail(SAGA_ERR_INVALID, "gemv: packed w must be 16-byte aligned");
-    if (M > 8) return fail(SAGA_ERR_UNSUPPORTED, "gemv: 8-row packed w takes at most 8 rows of x");
+  if (packed || packed8) {
+    if ((rc = check_packed(w, K))) return rc;
+    if (packed8 && M > 8) return fail(SAGA_ERR_UNSUPPORTED, "gemv: 8-row packed w takes at most 8 rows of x");
   } else if (w->shape[1] != K) {
     return fail(SAGA_ERR_INVALID, "gemv: w must be [N, K] with K = x.shape[1]");
   }
@@ -957,6 +963,41 @@ int saga_gemv(const saga_tensor* x, const saga_tensor* w, const saga_tensor* bia
     p.part_ssq = reinterpret_cast<float*>(static_cast<char*>(workspace) + align256(int64_t(splits) * p.M * p.N * 4));
   }
   if ((rc = hip_status(launch_gemv(p, static_cast<hipStream_t>(stream)), "gemv launch"))) return rc;
+  return ok();
+}
+
+int saga_unpack_gemv(const saga_unpack_item* items, int32_t n, saga_stream_t stream) {
+  if (!items || n < 1 || n > SAGA_UNPACK_MAX)
+    return fail(SAGA_ERR_INVALID, "unpack: 1 to %d items required", SAGA_UNPACK_MAX);
+  UnpackParams p{};
+  p.n = n;
+  for (int32_t i = 0; i < n; ++i) {
+    const saga_unpack_item& it = items[i];
+    int rc;
+    if (it.w.ndim != 3 && it.w.ndim != 4) return fail(SAGA_ERR_INVALID, "unpack: w must be a packed weight");
+    if ((rc = check_tensor(&it.w, "w", it.w.ndim)) || (rc = check_tensor(&it.out, "out", 2))) return rc;
+    if (it.w.dtype != SAGA_DTYPE_BF16 || it.out.dtype != SAGA_DTYPE_BF16)
+      return fail(SAGA_ERR_UNSUPPORTED, "unpack: bf16 only");
+    const int64_t N = it.out.shape[0], K = it.out.shape[1];
+    if ((rc = check_packed(&it.w, K))) return rc;
+    if (it.w.shape[0] * (it.w.ndim == 4 ? 16 : 8) != N) return fail(SAGA_ERR_INVALID, "unpack: out must be [N, K] of w");
+    if ((rc = check_vec_rows(&it.out, "out"))) return rc;
+    if (it.rot_heads < 0 || it.head_rows < 0 ||
+        (it.head_rows > 0 && (it.head_rows % 2 || N % it.head_rows || it.rot_heads > N / it.head_rows)))
+      return fail(SAGA_ERR_INVALID, "unpack: head_rows must be even and divide N, rot_heads at most N / head_rows");
+    if (N >= (1LL << 30) || K >= (1LL << 30)) return fail(SAGA_ERR_UNSUPPORTED, "unpack: sizes too large");
+    UnpackParams::Item& d = p.item[i];
+    d.src = it.w.data;
+    d.dst = it.out.data;
+    d.dst_ld = it.out.stride[0];
+    d.N = static_cast<int32_t>(N);
+    d.K = static_cast<int32_t>(K);
+    d.tile_rows = it.w.ndim == 4 ? 16 : 8;
+    d.rot_heads = static_cast<int32_t>(it.rot_heads);
+    d.head_rows = static_cast<int32_t>(it.head_rows);
+  }
+  int rc;
+  if ((rc = hip_status(launch_unpack(p, static_cast<hipStream_t>(stream)), "unpack launch"))) return rc;
   return ok();
 }
 

@@ -233,6 +233,21 @@ struct RowParams {
 hipError_t launch_rmsnorm(const RowParams& p, hipStream_t st);
 hipError_t launch_silu_mul(const RowParams& p, hipStream_t st);
 
+// Packed weights to row-major, up to kUnpackMax per launch.
+constexpr int kUnpackMax = SAGA_UNPACK_MAX;
+struct UnpackParams {
+  struct Item {
+    const void* src;
+    void* dst;
+    int64_t dst_ld;
+    int32_t N, K, tile_rows;
+    int32_t rot_heads, head_rows;  // head_rows 0: rows keep their order
+    int32_t block0;                // first block (set by the launcher)
+  } item[kUnpackMax];
+  int32_t n;
+};
+hipError_t launch_unpack(UnpackParams& p, hipStream_t st);
+
 // Skinny GEMM y[m, n] = rms(x)[m] * sum_k x[m, k] W[n, k] (+ epilogue), m < 32.
 struct GemvParams {
   const void* x;  // bf16 [M, K]

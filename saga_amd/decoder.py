@@ -224,7 +224,6 @@ class SagaDecoder:
                 order = ops.rope_pair_order(s.n_q, s.n_k, s.n_v, s.head_dim, device=self.device)
                 self.kw_qkv = [w.index_select(0, order).contiguous() for w in self.kw_qkv]
                 self.kb_qkv = [b.index_select(0, order).contiguous() for b in self.b_qkv]
-                self._unpair = torch.argsort(order)
             self.kw_gu = []
             for l in range(s.layers):
                 w = (self.w_gu[l].float() * self.ln2[l].float()).to(self.dtype)
@@ -275,7 +274,8 @@ class SagaDecoder:
     @staticmethod
     def _unpack(w: torch.Tensor) -> torch.Tensor:
         """Row-major [N, K] of a packed weight: [N/16, K/32, 16, 32] or, in
-        8-row tiles, [N/8, K/64, 512] (ops.pack_gemv_weight)."""
+        8-row tiles, [N/8, K/64, 512], in torch (any device; the prefill uses
+        ops.unpack_gemv_weights)."""
         if w.dim() == 2:
             return w
         if w.dim() == 3:
@@ -285,15 +285,16 @@ class SagaDecoder:
         return w.permute(0, 2, 1, 3).reshape(n16 * 16, k32 * 32)
 
     def _prefill_layer(self, l: int):
-        """(norm-1 weight, w_qkv, b_qkv, qkv column order, w_o, norm-2 weight,
-        w_gu, gate/up interleaved) for the prefill of layer l: the row-major
-        originals, or, once released, the unpacked decode copies (norms
-        folded in, q/k rows in rotary-pair order, gate/up interleaved)."""
+        """(norm-1 weight, w_qkv, w_o, norm-2 weight, w_gu, w_d), row-major and
+        in natural row order, for the prefill of layer l: the originals, or,
+        once released, the decode copies unpacked (norms folded in)."""
+        s = self.shape
         if self.w_qkv is not None:
-            return self.ln1[l], self.w_qkv[l], self.b_qkv[l], None, self.w_o[l], self.ln2[l], self.w_gu[l], False
-        unpair = self._unpair if self.fuse_rope else None
-        return (self._ones, self._unpack(self.kw_qkv[l]), self.kb_qkv[l], unpair, self._unpack(self.kw_o[l]),
-                self._ones, self._unpack(self.kw_gu[l]), True)
+            return self.ln1[l], self.w_qkv[l], self.w_o[l], self.ln2[l], self.w_gu[l], self.w_d[l]
+        w_qkv, w_o, w_gu, w_d = ops.unpack_gemv_weights(
+            (self.kw_qkv[l], self.kw_o[l], self.kw_gu[l], self.kw_d[l]),
+            ((s.n_q + s.n_k, s.head_dim) if self.fuse_rope else None, None, (1, 2 * s.intermediate), None))
+        return self._ones, w_qkv, w_o, self._ones, w_gu, w_d
 
     # ------------------------------------------------------------------ prefill
     @torch.no_grad()
@@ -310,11 +311,9 @@ class SagaDecoder:
         zeros = torch.zeros(T, device=self.device, dtype=torch.int32)
         mod = _HeadGroups()
         for l in range(s.layers):
-            n1, w_qkv, b_qkv, unpair, w_o, n2, w_gu, interleaved = self._prefill_layer(l)
+            n1, w_qkv, w_o, n2, w_gu, w_d = self._prefill_layer(l)
             h = ops.rmsnorm(x, n1, s.eps)
-            qkv = torch.addmm(b_qkv, h, w_qkv.t())
-            if unpair is not None:
-                qkv = qkv.index_select(1, unpair)
+            qkv = torch.addmm(self.b_qkv[l], h, w_qkv.t())
             q = ops.rope_kv_append(qkv, s.n_q, s.n_k, s.n_v, s.rope_theta, pos, self.k_cache[l], self.v_cache[l],
                                    batch=zeros)
             k = self.k_cache[l, 0:1, :, :T]
@@ -323,19 +322,17 @@ class SagaDecoder:
             # operands, else torch SDPA (attention/attention.py:13-53)
             o, _ = sdpa_attention_forward(mod, q.transpose(0, 1).unsqueeze(0), k, v, None, is_causal=True)
             x = torch.addmm(x, o.reshape(T, s.n_q * d), w_o.t())
-            w_d = self.w_d[l] if self.w_d is not None else self._unpack(self.kw_d[l])
             for c0 in range(0, T, chunk):
                 xc = x[c0:c0 + chunk]
                 gu = torch.mm(ops.rmsnorm(xc, n2, s.eps), w_gu.t())
-                if interleaved:  # (gate_0, up_0, gate_1, ...) -> [gate | up]
-                    gu = gu.view(gu.shape[0], s.intermediate, 2).transpose(1, 2).reshape(gu.shape[0], -1)
                 xc.addmm_(ops.silu_mul(gu), w_d.t())
             del w_qkv, w_o, w_gu, w_d
         if self.lm_head is not None:
             last = ops.rmsnorm(x[-1:], self.ln_f, s.eps)
             first = torch.mm(last, self.lm_head.t()).argmax(dim=-1)
         else:
-            first = torch.mm(ops.rmsnorm(x[-1:], self._ones, s.eps), self._unpack(self.kw_lm).t()).argmax(dim=-1)
+            # the packed head as the decode step reads it: one row needs no row-major copy of the vocabulary
+            first = ops.gemv(x[-1:], self.kw_lm, rms_eps=s.eps, workspace=self.ws.get("gemv")).argmax(dim=-1)
         self.k_cache[:, 1:, :, :T] = self.k_cache[:, 0:1, :, :T]
         self.v_cache[:, 1:, :, :T] = self.v_cache[:, 0:1, :, :T]
         self.prompt_len = T

@@ -505,6 +505,32 @@ def pack_gemv_weight(w: torch.Tensor, tile_rows: int = 16) -> torch.Tensor:
     return w.reshape(N // 8, 8, K // 64, 2, 32).permute(0, 2, 3, 1, 4).reshape(N // 8, K // 64, 512).contiguous()
 
 
+def unpack_gemv_weights(weights, heads=None):
+    """Row-major [N, K] of packed weights (pack_gemv_weight), all in one
+    launch; a weight that is row-major already is returned as it is.
+    heads: per weight (rot_heads, head_rows) or None: the first rot_heads
+    heads of head_rows rows go from rotary-pair order to natural order (one
+    head of N rows: interleaved gate/up pairs to [gate | up])."""
+    dev = _need_gpu(*weights)
+    heads = heads or [None] * len(weights)
+    outs, items = [], []
+    for w, h in zip(weights, heads):
+        if w.dim() == 2:
+            if h is not None:
+                raise ValueError("saga_amd: only packed weights are reordered")
+            outs.append(w)
+            continue
+        n, k = (w.shape[0] * 16, w.shape[1] * 32) if w.dim() == 4 else (w.shape[0] * 8, w.shape[1] * 64)
+        out = torch.empty(n, k, dtype=w.dtype, device=dev)
+        rot, rows = h if h is not None else (0, 0)
+        items.append(_lib.UnpackItem(_lib.descriptor(w), _lib.descriptor(out), rot, rows))
+        outs.append(out)
+    if items:
+        _lib.check(_lib.load().saga_unpack_gemv((_lib.UnpackItem * len(items))(*items), len(items),
+                                                _lib.stream_of(weights[0])), "unpack_gemv")
+    return outs
+
+
 def _gemv_n(w: torch.Tensor) -> int:
     return w.shape[0] * {4: 16, 3: 8}.get(w.dim(), 1)
 
