@@ -1054,7 +1054,7 @@ int saga_prefill_attention(const saga_tensor* query, const saga_tensor* key, con
     return fail(SAGA_ERR_INVALID, "prefill: causal_offset out of range");
   if (!(scale > 0.f) || !std::isfinite(scale))
     return fail(SAGA_ERR_UNSUPPORTED, "prefill: scale must be positive and finite");
-  const int64_t nmb = prefill_query_blocks(Lq, static_cast<int>(d));
+  const int64_t nmb = prefill_query_blocks(b, q_h, Lq, Lk, static_cast<int>(d), mask != nullptr);
   if (nmb * q_h * b >= (1LL << 31)) return fail(SAGA_ERR_UNSUPPORTED, "prefill: grid too large");
   if ((rc = check_vec_rows(query, "query")) || (rc = check_vec_rows(key, "key")) || (rc = check_vec_rows(value, "value")))
     return rc;

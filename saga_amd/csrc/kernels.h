@@ -302,7 +302,13 @@ struct PrefillParams {
   int32_t causal_off;
   float scale;
 };
-int prefill_query_blocks(int64_t Lq, int d);
+// Waves per block, wave groups that split the keys (32 * nw / ks queries per
+// block), and query blocks per (batch, head).
+struct PrefillShape {
+  int nw, ks;
+};
+PrefillShape prefill_shape(int64_t b, int64_t q_h, int64_t Lq, int64_t Lk, int d, bool masked);
+int64_t prefill_query_blocks(int64_t b, int64_t q_h, int64_t Lq, int64_t Lk, int d, bool masked);
 hipError_t launch_prefill_attention(int dtype, int d, const PrefillParams& p, hipStream_t st);
 
 }  // namespace saga

@@ -178,3 +178,78 @@ def test_prefill_rejects_bad_operands():
     q96, k96, v96 = _inputs(9, 1, 4, 1, 2, 16, 16, 96)
     with pytest.raises(Exception, match="head_dim"):
         ops.prefill_attention(q96, k96, v96)
+
+
+def _ref64(q, k, v, rows, causal, off, mask=None):
+    """float64 attention of the given query rows: [b, len(rows), q_h, d]."""
+    n = q.shape[1]
+    k, v = (x.repeat_interleave(n // x.shape[1], 1).double() for x in (k, v))
+    x = torch.matmul(q[:, :, rows].double(), k.transpose(2, 3)) / q.shape[3] ** 0.5
+    if causal:
+        keep = torch.arange(k.shape[2], device=q.device)[None, :] <= rows[:, None] + off
+        x = x.masked_fill(~keep, float("-inf"))
+    if mask is not None:
+        m = mask[:, :, rows]
+        x = x.masked_fill(~m, float("-inf")) if m.dtype == torch.bool else x + m.double()
+    return torch.matmul(torch.softmax(x, -1).nan_to_num(0.0), v).transpose(1, 2)
+
+
+# one launch per rule of the block shape: keys split (short grids, and chains of 1536 keys), 4 waves (short chains,
+# d 64, below 8192 keys), 8 waves; lengths around the 64-key tile and the 128-key stage, queries and keys of unequal number
+@pytest.mark.parametrize("b,q_h,k_h,v_h,d,Lq,Lk,causal,off", [
+    (1, 2, 1, 1, 128, 1, 1, False, 0), (1, 3, 1, 3, 128, 129, 63, False, 0), (1, 4, 2, 1, 64, 65, 65, True, 0),
+    (1, 12, 1, 2, 128, 127, 129, True, 2), (1, 12, 1, 2, 128, 1537, 1537, True, 0), (2, 15, 1, 5, 64, 1600, 1600, True, 0),
+    (1, 12, 1, 2, 128, 70, 3011, False, 0), (1, 4, 1, 1, 64, 300, 1000, True, 700), (1, 4, 1, 1, 128, 300, 200, True, -150),
+    (8, 12, 1, 2, 128, 321, 321, True, 0), (8, 15, 1, 5, 64, 200, 257, False, 0), (3, 24, 2, 2, 128, 1100, 1100, True, 0),
+    (1, 12, 1, 2, 128, 8200, 8200, True, 0), (1, 16, 1, 1, 128, 4200, 8255, False, 0), (1, 15, 1, 5, 64, 8193, 8193, True, 0)])
+def test_prefill_block_shapes(b, q_h, k_h, v_h, d, Lq, Lk, causal, off):
+    g = torch.Generator(device="cuda").manual_seed(Lq + Lk)
+    q = torch.randn(b, Lq, q_h, d, generator=g, device="cuda").bfloat16().transpose(1, 2)
+    # caches longer than Lk whose other rows are NaN: nothing past Lk may count
+    cache = [torch.full((b, h, Lk + 130, d), float("nan"), device="cuda", dtype=torch.bfloat16) for h in (k_h, v_h)]
+    for c in cache:
+        c[:, :, :Lk] = torch.randn(c[:, :, :Lk].shape, generator=g, device="cuda").bfloat16()
+    k, v = (c[:, :, :Lk] for c in cache)
+    got = ops.prefill_attention(q, k, v, is_causal=causal, causal_offset=off)
+    rows = torch.cat([torch.arange(min(Lq, 96)), torch.arange(max(Lq - 200, min(Lq, 96)), Lq)]).cuda()
+    ref = _ref64(q, k, v, rows, causal, off)
+    out = got[:, rows].double()
+    # bf16 P and output: rel-L2 2e-3 as in the cases above, twice that as the bar
+    assert torch.isfinite(out).all() and ((out - ref).norm() / ref.norm().clamp(min=1e-9)).item() < 5e-3
+
+
+@pytest.mark.parametrize("kind", ["bool", "bytes", "half", "float", "strided"])
+@pytest.mark.parametrize("b,h,d,Lq,Lk", [(2, 4, 64, 130, 191), (1, 2, 128, 257, 257), (3, 3, 128, 33, 64), (2, 2, 64, 5, 7)])
+def test_prefill_mask_loads(kind, b, h, d, Lq, Lk):
+    """Each way a mask reaches the kernel, rows at odd addresses, tiles wholly hidden, wholly visible and mixed,
+    and queries that see nothing (0)."""
+    g = torch.Generator(device="cuda").manual_seed(Lk)
+    q, k, v = (torch.randn(b, h, L, d, generator=g, device="cuda").bfloat16() for L in (Lq, Lk, Lk))
+    keep = torch.rand(b, 1, Lq, Lk + 3, generator=g, device="cuda") < 0.5
+    keep[:, :, :, 64:128] = False
+    keep[:, :, : Lq // 2, :64] = True
+    keep[:, :, Lq // 3] = False
+    keep = keep[..., :Lk]
+    mask = keep
+    if kind == "bytes":  # any non-zero byte keeps, as a cast to bool does
+        mask = (keep.to(torch.uint8) * 5).view(torch.bool)
+    elif kind in ("half", "float"):
+        mask = torch.randn(keep.shape, generator=g, device="cuda").masked_fill(~keep, float("-inf"))
+        mask = mask.to(torch.bfloat16 if kind == "half" else torch.float32)
+    elif kind == "strided":
+        mask = keep.transpose(2, 3).contiguous().transpose(2, 3)
+    got = ops.prefill_attention(q, k, v, mask).double()
+    ref = _ref64(q, k, v, torch.arange(Lq, device="cuda"), False, 0, mask if kind in ("half", "float") else keep)
+    assert ((got - ref).norm() / ref.norm()).item() < 5e-3 and not got[:, Lq // 3].any()
+
+
+def test_prefill_far_rows():
+    """Key rows 8 MB and more apart: a stage's offsets no longer fit the 32-bit lane offsets."""
+    L, d = 90, 128
+    buf = torch.zeros(L, 1 << 22, device="cuda", dtype=torch.bfloat16)
+    k = buf[None, None, :, 64:64 + d]
+    k.normal_()
+    q, v = (torch.randn(1, n, L, d, device="cuda").bfloat16() for n in (2, 1))
+    got = ops.prefill_attention(q, k, v, is_causal=True).double()
+    ref = _ref64(q, k, v, torch.arange(L, device="cuda"), True, 0)
+    assert ((got - ref).norm() / ref.norm()).item() < 5e-3
