@@ -94,3 +94,37 @@ def test_full_einsum_forward_several_queries(dt, mask_kind):
     assert rel_l2(got, ref) < (1e-5 if dt == "f32" else 5e-3)
     if dt != "f32":
         assert np.max(np.abs(got - ref)) < 2e-2
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("b,q_h,k_h,v_h,d", [(4, 12, 2, 2, 128), (4, 12, 1, 2, 128), (4, 8, 2, 1, 128), (5, 15, 1, 5, 64),
+                                             (4, 16, 4, 8, 64), (2, 16, 1, 1, 64), (4, 12, 1, 3, 128)])
+@pytest.mark.parametrize("L", [1, 31, 33, 129, 1055])
+def test_dense_value_head_layouts(dt, b, q_h, k_h, v_h, d, L):
+    """Units of one, two and five whole value heads (MFMA) and others (VALU), at the edges of the 32-position step, with
+    ragged kv_len: cache rows past it are NaN (VALU: large) and one value head holds infinities, which reach its own
+    query heads only."""
+    import torch as T
+    g = T.Generator(device="cuda").manual_seed(L + q_h)
+    tdt = T.bfloat16 if dt == "bf16" else T.float16
+    q = T.randn(b, q_h, 1, d, generator=g, device="cuda").to(tdt)
+    k = T.randn(b, k_h, L + 40, d, generator=g, device="cuda").to(tdt)
+    v = T.randn(b, v_h, L + 40, d, generator=g, device="cuda").to(tdt)
+    lens = [max(1, L - 7 * i) for i in range(b)]
+    for i, n in enumerate(lens):
+        k[i, :, n:] = v[i, :, n:] = float("nan") if v_h != 3 else 100.0
+    if v_h != 3:
+        v[:, 0, 0] = float("inf")
+    kv = T.tensor(lens, dtype=T.int32, device="cuda")
+    out = ops.dense_decode(q, k[:, :, :L], v[:, :, :L], kv_len=kv, out_dtype=T.float32).double()
+    for i, n in enumerate(lens):
+        kk = k[i, :, :n].double().repeat_interleave(q_h // k_h, 0)
+        vv = v[i, :, :n].double().repeat_interleave(q_h // v_h, 0)
+        p = T.softmax((q[i].double() @ kk.transpose(1, 2)) / d ** 0.5, -1)
+        ref = (p @ vv)[:, 0]
+        own = T.arange(q_h) < q_h // v_h  # the query heads of value head 0
+        assert v_h == 3 or T.isinf(out[i, own, 0]).all()
+        if v_h > 1:
+            # exact products, fp32 sums and exp: 1e-6 relative and a few units per sum
+            got, want = out[i, ~own, 0], ref[~own]
+            assert T.isfinite(got).all() and ((got - want).norm() / want.norm()).item() < 1e-5
