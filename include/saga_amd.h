@@ -326,6 +326,12 @@ typedef struct saga_unpack_item {
 } saga_unpack_item;
 int saga_unpack_gemv(const saga_unpack_item* items, int32_t n, saga_stream_t stream);
 
+/* A prompt's gate/up projection with its activation, from the weight as the
+ * decode step keeps it: x [T, K] bf16, w packed [N/16, K/32, 16, 32] with rows
+ * interleaved (gate_i, up_i) as for SAGA_GEMV_SILU_PAIRS, K % 64 == 0;
+ * y[t, i] = silu(gate_i) * up_i, y [T, N / 2].  x and y rows 16-byte aligned. */
+int saga_prompt_mlp(const saga_tensor* x, const saga_tensor* w, saga_tensor* y, saga_stream_t stream);
+
 /* saga_gemv (STORE, bias, fused RMSNorm) of the fused q/k/v projection with
  * saga_rope_kv_append applied in its epilogue: one launch per layer for
  * projection + RoPE + cache append.  x [M, K] (M <= 32 new tokens), w bf16

@@ -80,6 +80,7 @@ _SIGS = {
     "saga_gemv_workspace_bytes": (ctypes.c_size_t, [_I64, _I64, _I64]),
     "saga_gemv": (ctypes.c_int, [_T, _T, _T, ctypes.c_float, ctypes.c_int32, _T, _P, ctypes.c_size_t, _P]),
     "saga_unpack_gemv": (ctypes.c_int, [ctypes.POINTER(UnpackItem), ctypes.c_int32, _P]),
+    "saga_prompt_mlp": (ctypes.c_int, [_T, _T, _T, _P]),
     "saga_gemv_rope_kv": (ctypes.c_int, [_T, _T, _T, ctypes.c_float, _I64, _I64, _I64, ctypes.c_float, _P, _P,
                                          _T, _T, _T, _P, _P]),
     "saga_rope_table": (ctypes.c_int, [_P, _I64, _I64, ctypes.c_float, _P, _P]),

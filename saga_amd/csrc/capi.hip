@@ -1001,6 +1001,31 @@ int saga_unpack_gemv(const saga_unpack_item* items, int32_t n, saga_stream_t str
   return ok();
 }
 
+int saga_prompt_mlp(const saga_tensor* x, const saga_tensor* w, saga_tensor* y, saga_stream_t stream) {
+  int rc;
+  if ((rc = check_tensor(x, "x", 2)) || (rc = check_tensor(w, "w", 4)) || (rc = check_tensor(y, "y", 2))) return rc;
+  if (x->dtype != SAGA_DTYPE_BF16 || w->dtype != SAGA_DTYPE_BF16 || y->dtype != SAGA_DTYPE_BF16)
+    return fail(SAGA_ERR_UNSUPPORTED, "prompt_mlp: bf16 only");
+  const int64_t T = x->shape[0], K = x->shape[1], N = w->shape[0] * 16;
+  if ((rc = check_packed(w, K))) return rc;
+  if (y->shape[0] != T || y->shape[1] != N / 2) return fail(SAGA_ERR_INVALID, "prompt_mlp: y must be [T, N / 2]");
+  if (K % 64 || K >= (1LL << 24)) return fail(SAGA_ERR_UNSUPPORTED, "prompt_mlp: K %% 64 == 0 required");
+  if (T >= (1LL << 24) || N >= (1LL << 24)) return fail(SAGA_ERR_UNSUPPORTED, "prompt_mlp: sizes too large");
+  if ((rc = check_vec_rows(x, "x")) || (rc = check_vec_rows(y, "y"))) return rc;
+  if (T == 0 || N == 0 || K == 0) return T && N ? fail(SAGA_ERR_INVALID, "prompt_mlp: K must be positive") : ok();
+  PromptMlpParams p{};
+  p.x = x->data;
+  p.w = w->data;
+  p.y = y->data;
+  p.x_ld = x->stride[0];
+  p.y_ld = y->stride[0];
+  p.T = static_cast<int32_t>(T);
+  p.N = static_cast<int32_t>(N);
+  p.K = static_cast<int32_t>(K);
+  if ((rc = hip_status(launch_prompt_mlp(p, static_cast<hipStream_t>(stream)), "prompt_mlp launch"))) return rc;
+  return ok();
+}
+
 size_t saga_argmax_workspace_bytes(int64_t rows, int64_t N) {
   if (rows < 1 || N < 1 || rows >= (1LL << 31) || N >= (1LL << 31)) return 0;
   return static_cast<size_t>(argmax_workspace_bytes(rows, N));

@@ -281,6 +281,18 @@ hipError_t launch_gemv(const GemvParams& p, hipStream_t st);
 int64_t argmax_workspace_bytes(int64_t rows, int64_t N);
 hipError_t launch_argmax(const void* x, int64_t ld, int rows, int N, int64_t* out, void* ws, hipStream_t st);
 
+// A prompt's gate/up projection and activation from the packed decode weight
+// (csrc/prompt_mlp.hip): x [T, K], w [N/16][K/32][16][32], y [T, N / 2].
+struct PromptMlpParams {
+  const void* x;
+  const void* w;
+  void* y;
+  int64_t x_ld, y_ld;
+  int32_t T, N, K;
+  int32_t mtiles, ntiles;  // set at launch
+};
+hipError_t launch_prompt_mlp(const PromptMlpParams& p, hipStream_t st);
+
 // Prefill attention with separate key / value head maps (csrc/prefill.hip).
 // Strides in elements; q [b, q_h, Lq, d], k [b, k_h, Lk, d], v [b, v_h, Lk, d],
 // mask [b|1, q_h|1, Lq, Lk] (broadcast dims stride 0), out [b, Lq, q_h, d].

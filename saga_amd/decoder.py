@@ -287,13 +287,20 @@ class SagaDecoder:
     def _prefill_layer(self, l: int):
         """(norm-1 weight, w_qkv, w_o, norm-2 weight, w_gu, w_d), row-major and
         in natural row order, for the prefill of layer l: the originals, or,
-        once released, the decode copies unpacked (norms folded in)."""
+        once released, the decode copies unpacked (norms folded in); w_gu None
+        where ops.prompt_mlp takes the packed copy."""
         s = self.shape
         if self.w_qkv is not None:
             return self.ln1[l], self.w_qkv[l], self.w_o[l], self.ln2[l], self.w_gu[l], self.w_d[l]
-        w_qkv, w_o, w_gu, w_d = ops.unpack_gemv_weights(
-            (self.kw_qkv[l], self.kw_o[l], self.kw_gu[l], self.kw_d[l]),
-            ((s.n_q + s.n_k, s.head_dim) if self.fuse_rope else None, None, (1, 2 * s.intermediate), None))
+        weights = [self.kw_qkv[l], self.kw_o[l], self.kw_d[l]]
+        heads = [(s.n_q + s.n_k, s.head_dim) if self.fuse_rope else None, None, None]
+        w_gu = None  # ops.prompt_mlp reads the packed weight
+        if not ops.prompt_mlp_supported(self.kw_gu[l]):
+            weights.append(self.kw_gu[l])
+            heads.append((1, 2 * s.intermediate))
+        w_qkv, w_o, w_d, *rest = ops.unpack_gemv_weights(weights, heads)
+        if rest:
+            w_gu = rest[0]
         return self._ones, w_qkv, w_o, self._ones, w_gu, w_d
 
     # ------------------------------------------------------------------ prefill
@@ -321,11 +328,12 @@ class SagaDecoder:
             # the HIP prefill kernel when ops.prefill_supported holds for these
             # operands, else torch SDPA (attention/attention.py:13-53)
             o, _ = sdpa_attention_forward(mod, q.transpose(0, 1).unsqueeze(0), k, v, None, is_causal=True)
-            x = torch.addmm(x, o.reshape(T, s.n_q * d), w_o.t())
+            x.addmm_(o.reshape(T, s.n_q * d), w_o.t())
             for c0 in range(0, T, chunk):
                 xc = x[c0:c0 + chunk]
-                gu = torch.mm(ops.rmsnorm(xc, n2, s.eps), w_gu.t())
-                xc.addmm_(ops.silu_mul(gu), w_d.t())
+                h = ops.rmsnorm(xc, n2, s.eps)
+                act = ops.prompt_mlp(h, self.kw_gu[l]) if w_gu is None else ops.silu_mul(torch.mm(h, w_gu.t()))
+                xc.addmm_(act, w_d.t())
             del w_qkv, w_o, w_gu, w_d
         if self.lm_head is not None:
             last = ops.rmsnorm(x[-1:], self.ln_f, s.eps)

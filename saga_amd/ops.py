@@ -531,6 +531,21 @@ def unpack_gemv_weights(weights, heads=None):
     return outs
 
 
+def prompt_mlp_supported(w: torch.Tensor) -> bool:
+    """Whether prompt_mlp takes a gate/up weight: packed in 16-row tiles, K a multiple of its 64-wide steps."""
+    return w.dim() == 4 and w.dtype == torch.bfloat16 and w.shape[1] % 2 == 0
+
+
+def prompt_mlp(x, w, out=None):
+    """silu(gate) * up of a prompt's rows x [T, K] for w packed by
+    pack_gemv_weight from interleaved gate/up rows [N, K] -> [T, N / 2]."""
+    dev = _need_gpu(x, w, out)
+    out = torch.empty(x.shape[0], w.shape[0] * 8, dtype=x.dtype, device=dev) if out is None else out
+    _lib.check(_lib.load().saga_prompt_mlp(_lib.tensor(x), _lib.tensor(w), _lib.tensor(out), _lib.stream_of(x)),
+               "prompt_mlp")
+    return out
+
+
 def _gemv_n(w: torch.Tensor) -> int:
     return w.shape[0] * {4: 16, 3: 8}.get(w.dim(), 1)
 
