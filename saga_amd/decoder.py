@@ -337,7 +337,13 @@ class SagaDecoder:
             del w_qkv, w_o, w_gu, w_d
         if self.lm_head is not None:
             last = ops.rmsnorm(x[-1:], self.ln_f, s.eps)
-            first = torch.mm(last, self.lm_head.t()).argmax(dim=-1)
+            head = self.lm_head
+            if head.dtype == torch.bfloat16 and head.is_contiguous() and head.data_ptr() % 16 == 0 \
+                    and head.shape[0] % 16 == 0 and s.hidden % 32 == 0:
+                # one row: the weight stream of the decode step (466 MB: 161 us in the library's GEMM)
+                first = ops.gemv(last, head, split_k=False).argmax(dim=-1)
+            else:
+                first = torch.mm(last, head.t()).argmax(dim=-1)
         else:
             # the packed head as the decode step reads it: one row needs no row-major copy of the vocabulary
             first = ops.gemv(x[-1:], self.kw_lm, rms_eps=s.eps, workspace=self.ws.get("gemv")).argmax(dim=-1)
