@@ -289,7 +289,7 @@ struct PromptMlpParams {
   void* y;
   int64_t x_ld, y_ld;
   int32_t T, N, K;
-  int32_t mtiles, ntiles;  // set at launch
+  int32_t mtiles, ntiles, whole;  // set at launch
 };
 hipError_t launch_prompt_mlp(const PromptMlpParams& p, hipStream_t st);
 

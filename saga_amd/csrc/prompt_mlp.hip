@@ -10,9 +10,9 @@
 // fragment reads meet in a bank.  gate and up meet in one lane, so the
 // [T, N] projection never exists in memory and W is not unpacked first.
 // Against unpacking W, the library GEMM and silu_mul (one box, us): N 17920,
-// K 1536: 4001 tokens 230 -> 209 (1.05 PFLOP/s; 5 rounds of blocks for 4.4
-// rounds of work), 8192 458 -> 388, 1500 108 -> 84, 700 72 -> 44, 128
-// 41 -> 19; N 5120, K 960: 4001 75 -> 55, 512 38 -> 13.
+// K 1536: 4001 tokens 239 -> 198 (1.11 PFLOP/s), 8192 451 -> 381, 1500
+// 107 -> 84, 700 65 -> 40, 128 41 -> 19; N 5120, K 960: 4001 73 -> 49, 512
+// 39 -> 13.
 #include <algorithm>
 
 #include "common.cuh"
@@ -27,31 +27,26 @@ constexpr int kXcds = 8;
 constexpr int64_t kCus = 256;
 constexpr int kMlpGroup = 8;  // token tiles that share a sweep over W (their x and the W tiles stay in an XCD's L2)
 
+// LDS of a block: two x buffers, or the output rows (TN / 2 values, padded).
+template <int MF, int NF>
+constexpr int mlp_lds() {
+  constexpr int x = 2 * 32 * MF * kMlpStep * 2, out = 32 * MF * (64 * NF + 16);
+  return x > out ? x : out;
+}
+
+// Tokens from t0, W rows from n0.
 template <int MF, int NF, int D>
-__global__ void __launch_bounds__(kMlpThreads, 2) prompt_mlp_kernel(PromptMlpParams p) {
+__device__ __forceinline__ void mlp_block(const PromptMlpParams& p, int t0, int n0, char* lds) {
   constexpr int TM = 32 * MF, TN = 64 * NF;
   constexpr int NX = TM / 64;                // 16-byte units of x per thread and step
   constexpr int kLoads = NX + 2 * NF;        // global loads per step
   constexpr int XBYTES = TM * kMlpStep * 2;  // one x buffer
-  constexpr int OROW = TN + 16;              // bytes of an output row in LDS (TN / 2 values, padded)
-  constexpr int LDS = 2 * XBYTES > TM * OROW ? 2 * XBYTES : TM * OROW;
-  __shared__ __attribute__((aligned(16))) char lds[LDS];
+  constexpr int OROW = TN + 16;              // bytes of an output row in LDS
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, s = lane >> 4;
   const int wm = w & 1, wn = w >> 1;
 
-  // Blocks go to the XCDs round robin: XCD i takes the i-th contiguous part
-  // of the tile list (groups of kMlpGroup token tiles, W tiles within).
-  const int total = p.mtiles * p.ntiles;
-  const int xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
-  const int base = total / kXcds, rem = total % kXcds;
-  const int tile = xcd * base + min(xcd, rem) + slot;
-  const int gsize = kMlpGroup * p.ntiles;
-  const int grp = tile / gsize, in = tile - grp * gsize;
-  const int gm = min(kMlpGroup, p.mtiles - grp * kMlpGroup);
-  const int nt = in / gm, mt = grp * kMlpGroup + in - nt * gm;
-  const int t0 = mt * TM, n0 = nt * TN;
   const int ksteps = p.K / kMlpStep;
 
   // x: unit i of the thread is k chunk c (8 values) of token row r
@@ -162,12 +157,52 @@ __global__ void __launch_bounds__(kMlpThreads, 2) prompt_mlp_kernel(PromptMlpPar
   }
 }
 
+// Position of block b of n in the tile list: blocks go to the XCDs round
+// robin, XCD i takes the i-th contiguous part.
+__device__ __forceinline__ int xcd_tile(int b, int n) {
+  const int xcd = b % kXcds, rem = n % kXcds;
+  return xcd * (n / kXcds) + min(xcd, rem) + b / kXcds;
+}
+
+// Token and W tile of entry i of the list (groups of kMlpGroup token tiles, W
+// tiles within).
+__device__ __forceinline__ void list_tile(const PromptMlpParams& p, int i, int& mt, int& nt) {
+  const int gsize = kMlpGroup * p.ntiles;
+  const int grp = i / gsize, in = i - grp * gsize;
+  const int gm = min(kMlpGroup, p.mtiles - grp * kMlpGroup);
+  nt = in / gm;
+  mt = grp * kMlpGroup + in - nt * gm;
+}
+
+// One block per tile of the list for the first p.whole tiles, then (NF even)
+// two blocks per tile, one half of its W rows each: the last round's tiles
+// when they would leave half the CUs idle.
 template <int MF, int NF, int D>
-hipError_t launch_shape(PromptMlpParams p, hipStream_t st) {
+__global__ void __launch_bounds__(kMlpThreads, 2) prompt_mlp_kernel(PromptMlpParams p) {
+  __shared__ __attribute__((aligned(16))) char lds[mlp_lds<MF, NF>()];
+  const int b = blockIdx.x;
+  int mt, nt;
+  if constexpr (NF == 4) {
+    if (b >= p.whole) {
+      const int h = xcd_tile(b - p.whole, gridDim.x - p.whole);
+      list_tile(p, p.whole + h / 2, mt, nt);
+      const int n0 = nt * 64 * NF + (h & 1) * 32 * NF;
+      if (n0 < p.N) mlp_block<MF, NF / 2, D>(p, mt * 32 * MF, n0, lds);
+      return;
+    }
+  }
+  list_tile(p, xcd_tile(b, p.whole), mt, nt);
+  mlp_block<MF, NF, D>(p, mt * 32 * MF, nt * 64 * NF, lds);
+}
+
+template <int MF, int NF, int D>
+hipError_t launch_shape(PromptMlpParams p, bool halves, hipStream_t st) {
   p.mtiles = (p.T + 32 * MF - 1) / (32 * MF);
   p.ntiles = (p.N + 64 * NF - 1) / (64 * NF);
-  hipLaunchKernelGGL((prompt_mlp_kernel<MF, NF, D>), dim3(static_cast<unsigned>(p.mtiles * p.ntiles)), dim3(kMlpThreads), 0,
-                     st, p);
+  const int total = p.mtiles * p.ntiles;
+  p.whole = halves ? total / kCus * kCus : total;
+  hipLaunchKernelGGL((prompt_mlp_kernel<MF, NF, D>), dim3(static_cast<unsigned>(2 * total - p.whole)),
+                     dim3(kMlpThreads), 0, st, p);
   return hipGetLastError();
 }
 
@@ -179,13 +214,18 @@ hipError_t launch_prompt_mlp(const PromptMlpParams& p, hipStream_t st) {
   // 256 x 128 25, of 128 x 128 (loads three steps ahead, in the registers
   // that its products leave) 18.5: ratios 8, 5.6 and 4.1.  64-token blocks
   // took as long as 128-token ones; 128 x 256 31 us.
-  auto rounds = [&](int tm, int tn) {
-    return (static_cast<int64_t>((p.T + tm - 1) / tm) * ((p.N + tn - 1) / tn) + kCus - 1) / kCus;
-  };
-  const int64_t c84 = 80 * rounds(256, 256), c82 = 56 * rounds(256, 128), c42 = 41 * rounds(128, 128);
-  if (c42 <= c82 && c42 <= c84) return launch_shape<4, 2, 3>(p, st);
-  if (c82 < c84) return launch_shape<8, 2, 1>(p, st);
-  return launch_shape<8, 4, 1>(p, st);
+  // After a whole round of 256 x 256 blocks a rest of at most half a round
+  // goes as 256 x 128 blocks (N 17920: 1000 tokens, 280 tiles, 77 -> 66 us;
+  // 4001, 1120 tiles, 212 -> 198).
+  auto tiles = [&](int tm, int tn) { return static_cast<int64_t>((p.T + tm - 1) / tm) * ((p.N + tn - 1) / tn); };
+  auto rounds = [&](int64_t n) { return (n + kCus - 1) / kCus; };
+  const int64_t n84 = tiles(256, 256), rest = n84 % kCus;
+  const bool halves = n84 > kCus && rest > 0 && 2 * rest <= kCus;
+  const int64_t c84 = halves ? 80 * (n84 / kCus) + 56 : 80 * rounds(n84);
+  const int64_t c82 = 56 * rounds(tiles(256, 128)), c42 = 41 * rounds(tiles(128, 128));
+  if (c42 <= c82 && c42 <= c84) return launch_shape<4, 2, 3>(p, false, st);
+  if (c82 < c84) return launch_shape<8, 2, 1>(p, false, st);
+  return launch_shape<8, 4, 1>(p, halves, st);
 }
 
 }  // namespace saga

@@ -8,9 +8,11 @@ pytestmark = pytest.mark.gpu
 
 # token counts at the edges of a block (128 and 256 tokens), weights of one tile and of a partial last block (128 and
 # 256 rows), one k step, odd and even numbers of them; the launch takes blocks of 128 x 128 but for (700, 17936) and
-# (2500, 4112): 256 x 256, and (2111, 2576): 256 x 128
+# (2500, 4112): 256 x 256, (2111, 2576): 256 x 128, and (1000, 17936), (2100, 7952): 256 x 256 with a
+# rest in halves, the second with a last half past the weight's rows
 CASES = [(1, 16, 64), (17, 144, 192), (64, 5120, 960), (65, 272, 128), (128, 640, 64), (129, 5136, 320), (512, 1008, 448),
-         (513, 272, 1536), (768, 5136, 192), (700, 17936, 192), (2500, 4112, 64), (2111, 2576, 960)]
+         (513, 272, 1536), (768, 5136, 192), (700, 17936, 192), (2500, 4112, 64), (2111, 2576, 960),
+         (1000, 17936, 128), (2100, 7952, 64)]
 
 
 @pytest.mark.parametrize("T,N,K", CASES)
