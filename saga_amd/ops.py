@@ -114,6 +114,12 @@ def _scale(query: torch.Tensor, scaling: Optional[float]) -> float:
 def _vec_ready(t: torch.Tensor) -> torch.Tensor:
     """Rows must have a unit innermost stride and 16-byte aligned strides."""
     es = t.element_size()
+    if t.dim() == 4:
+        # the usual case, without the loop: every stride a multiple of 16 bytes whatever its size
+        # (an or of strides is a multiple of a power of two exactly when each of them is)
+        s0, s1, s2, s3 = t.stride()
+        if s3 == 1 and ((s0 | s1 | s2) * es | t.data_ptr()) % 16 == 0:
+            return t
     ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(
         (s * es) % 16 == 0 for s, n in zip(t.stride()[:-1], t.shape[:-1]) if n > 1)
     return t if ok else t.contiguous()
