@@ -90,7 +90,11 @@ __device__ __forceinline__ void mlp_block(const PromptMlpParams& p, int t0, int 
   // load, 96 loads) and every wave waits there with its products undone.  The
   // step's own x is in LDS; the next step's goes into the other buffer last
   // (read by every wave before this step's barrier).
-  constexpr int kAhead = F < 4 ? F : 4;
+  // 4001 tokens, 17920 x 1536: loads at the step's start 250 us, spread 209
+  // (both with five whole rounds of blocks); then 190 with 4 fragments ahead,
+  // 188 with 3 (no more than boxes differ), 203 with 6 (spills), 226 without
+  // the scheduling fences between the fragments.
+  constexpr int kAhead = 4;
   auto step = [&](int k, int st) {
     lds_sync();
     const int kn = min(k + D, ksteps - 1), sn = (st + D) % R;
