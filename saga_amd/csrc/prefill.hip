@@ -173,9 +173,9 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
   const int kst = pf_krow(lr) * S::KROW + 4 * lc;  // and kstep dwords per RPP (16, 32 or 64) rows
   constexpr int kstep = S::RPP * S::KROW;
   static_assert(S::RPP % 16 == 0, "pf_krow permutes within 16 rows");
-  // Rows outside the cache repeat its first or last row (the length mask gives
-  // rows at or past Lk weight 0) and stages past the last are loaded but never
-  // read, so that no load sits under a branch (900 cycles a stage); scalar
+  // Rows outside the cache repeat its first or last row (rows at or past Lk get
+  // weight 0 from the length mask and zero values from zero_tail) and stages past
+  // the last are loaded but never read, so that no load sits under a branch (900 cycles a stage); scalar
   // bases and one 32-bit offset per lane keep 64-bit address arithmetic off the
   // vector unit (20 % of the whole kernel when each load did its own).
   const bool near = krow < (1 << 23) && vrow < (1 << 23);  // a stage's offsets fit 32 bits
@@ -198,6 +198,16 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
   auto load_stage = [&](int st) {
     load_rows(kb, krow, st * S::BNS, kr);
     load_rows(vb, vrow, (st - 1) * S::BNS, vr);
+  };
+  // V rows of stage st at or past Lk are copies of the last row: their weight
+  // is 0, but 0 * inf is NaN, so zeros are staged in their place.  No stage
+  // that load_stage_full loads has such rows.
+  auto zero_tail = [&](int st) {
+    const int r0 = (st - 1) * S::BNS;
+    if (r0 + S::BNS <= p.Lk) return;
+#pragma unroll
+    for (int i = 0; i < S::KPT; ++i)
+      if (r0 + lr + i * S::RPP >= p.Lk) vr[i] = u32x4{0u, 0u, 0u, 0u};
   };
   // the next stage of a run of stages whose K rows lie below Lk, near
   const char* kcur = kb + 3 * S::BNS * krow + koffs;
@@ -447,6 +457,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
     if (second) lds_sync();  // the second half runs one phase behind the first; a barrier ends every phase
     bool vis = nmine > 0 && mask_visible();
     if (vis) qk(0);
+    zero_tail(1);
     write_stage(1);
     load_stage(2);
     if constexpr (kPing) lds_sync();
@@ -467,6 +478,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
       if (vis) pv(it + 1);
       const bool next = it + 1 < nmine && mask_visible();
       if (next) qk(it + 1);
+      zero_tail(it + 2);
       write_stage(it + 2);
       load_stage(it + 3);
       vis = next;
@@ -474,6 +486,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
     }
     for (; it < ntiles; ++it) {  // keys only the block's later waves see
       lds_sync();
+      zero_tail(it + 2);
       write_stage(it + 2);
       load_stage(it + 3);
       if constexpr (kPing) lds_sync();

@@ -253,3 +253,35 @@ def test_prefill_far_rows():
     got = ops.prefill_attention(q, k, v, is_causal=True).double()
     ref = _ref64(q, k, v, torch.arange(L, device="cuda"), True, 0)
     assert ((got - ref).norm() / ref.norm()).item() < 5e-3
+
+
+# the split-key, 4-wave and 8-wave blocks; lengths one past a 64-key tile (a stage filled up with repeated rows) and,
+# for comparison, whole tiles
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["full", "causal", "bool", "half", "float"])
+@pytest.mark.parametrize("b,q_h,Lq,Lk,d", [(1, 4, 70, 65, 64), (1, 4, 70, 65, 128), (2, 4, 33, 129, 64), (1, 4, 130, 129, 128),
+                                           (1, 4, 70, 128, 128), (11, 12, 130, 129, 64), (11, 12, 130, 65, 128),
+                                           (22, 12, 1, 8193, 128)])
+def test_prefill_infinite_last_value(b, q_h, Lq, Lk, d, kind, dt):
+    """An infinite value in the last key row makes that dim infinite for the queries that see the row: what a partial
+    tile is filled up with has weight 0 and must not meet it."""
+    g = torch.Generator(device="cuda").manual_seed(Lk + d)
+    q, k, v = (torch.randn(b, h, L, d, generator=g, device="cuda").to(dt) for h, L in ((q_h, Lq), (1, Lk), (2, Lk)))
+    v[:, 0, -1, 5], v[:, 1, -1, 6] = float("inf"), -float("inf")
+    mask = None
+    if kind in ("bool", "half", "float"):
+        mask = torch.rand(b, 1, Lq, Lk, generator=g, device="cuda") < 0.7
+        mask[..., -1] = True
+        if kind != "bool":
+            mask = torch.zeros(mask.shape, device="cuda").masked_fill(~mask, -float("inf"))
+            mask = mask.to(dt) if kind == "half" else mask
+    causal = kind == "causal"  # its last query sees the last key, the others do not
+    got = ops.prefill_attention(q, k, v, mask, is_causal=causal, causal_offset=Lk - Lq if causal else 0)
+    rows = torch.arange(Lq - 1 if causal else 0, Lq, device="cuda")
+    ref = _ref64(q, k, v, rows, causal, Lk - Lq if causal else 0, mask)
+    out, half = got[:, rows].double(), q_h // 2
+    assert (out[:, :, :half, 5] == float("inf")).all() and (out[:, :, half:, 6] == -float("inf")).all()
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(out), fin)
+    # 16-bit P and output, as in the cases above
+    assert ((out[fin] - ref[fin]).norm() / ref[fin].norm()).item() < 5e-3
