@@ -306,8 +306,11 @@ struct DenseMfma {
 // consecutive keys of its head: the B operand of the second product), V rows
 // through wave-private LDS, read transposed (ds_read_b64_tr_b16: 4 keys of
 // one dim) as the A operand of O^T += V^T P^T.  P stays 32 bits: it is split
-// exactly into three 16-bit terms, three MFMAs (24 bits).  A head's output
-// column only takes its own value head's sums.
+// exactly into 16-bit terms, an MFMA each: three of bf16 (24 bits).  f16 ends
+// at 2^-24, so P is held times 2^15, where three terms are exact for weights
+// from 2^-16 on, and a step with smaller ones adds terms in smaller units
+// until nothing is left of them.  A head's output column only takes its own
+// value head's sums.
 //
 // Bound by the K + V stream, so the registers of a step's loads are emptied
 // (QK, LDS write) and refilled with the next step's before its softmax and
@@ -325,6 +328,8 @@ __global__ void __launch_bounds__(256, 2) dense_mfma_kernel(DenseParams p) {
   constexpr int NVL = 32 / RPL;       // loads per value head and step
   constexpr int NDT = D / 16;
   constexpr uint16_t kInf16 = DT == SAGA_DTYPE_BF16 ? 0x7f80 : 0x7c00;
+  constexpr bool kF16 = DT == SAGA_DTYPE_F16;
+  constexpr float kTop = 32768.f;  // f16: P and o are held times this
   __shared__ __attribute__((aligned(16))) uint32_t lds[S::LDS];
 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -460,6 +465,10 @@ __global__ void __launch_bounds__(256, 2) dense_mfma_kernel(DenseParams p) {
     constexpr uint32_t kOne = DT == SAGA_DTYPE_BF16 ? 0x3f80u : 0x3c00u;
 #pragma unroll
     for (int i = 0; i < 4; ++i) some[i] = (x[2 * i] > 0.f ? kOne : 0u) | (x[2 * i + 1] > 0.f ? kOne << 16 : 0u);
+    if constexpr (kF16) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] *= kTop;
+    }
     u32x4 pf[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k)
@@ -478,6 +487,35 @@ __global__ void __launch_bounds__(256, 2) dense_mfma_kernel(DenseParams p) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) o[u][dt] = mfma_16b<DT>(vf, pf[k], o[u][dt]);
       }
+    if constexpr (kF16) {
+      // what f16 terms in the first unit leave of weights below 2^-16, at most 2^-25: in a unit 2^40 times smaller, and
+      // then in steps of 2^12 (8 terms reach the last bit of the smallest float; a NaN leaves nothing)
+      float unit = 1.f;
+#pragma unroll 1  // a peeled pass spills
+      for (int k = 0; k < 8; ++k) {
+        bool left = false;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) left |= x[i] > 0.f || x[i] < 0.f;
+        if (!__any(left)) break;
+        const float up = k == 0 ? 0x1p40f : 0x1p12f;
+        unit *= k == 0 ? 0x1p-40f : 0x1p-12f;
+        u32x4 pt;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          x[2 * i] *= up;
+          x[2 * i + 1] *= up;
+          pt[i] = split2<DT>(x[2 * i], x[2 * i + 1]);
+        }
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+#pragma unroll
+          for (int dt = 0; dt < NDT; ++dt) {
+            const f32x4 t = mfma_16b<DT>(v_frag(u, dt), pt, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[u][dt][e] = __builtin_fmaf(t[e], unit, o[u][dt][e]);
+          }
+      }
+    }
     if (special) {  // weight > 0: inf, -inf or NaN; weight 0: NaN
       dense_wave_sync();
       for (int i = 0; i < NVL; ++i) {
@@ -510,6 +548,7 @@ __global__ void __launch_bounds__(256, 2) dense_mfma_kernel(DenseParams p) {
     f32x4 a = o[0][dt];
 #pragma unroll
     for (int u = 1; u < NV; ++u) a = u_mine == u ? o[u][dt] : a;
+    if constexpr (kF16) a *= 1.f / kTop;
     *reinterpret_cast<f32x4*>(Wo + (w * 16 + col) * S::WROW + 16 * dt + 4 * s) = a;
   }
   __syncthreads();

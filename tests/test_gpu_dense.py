@@ -128,3 +128,28 @@ def test_dense_value_head_layouts(dt, b, q_h, k_h, v_h, d, L):
             # exact products, fp32 sums and exp: 1e-6 relative and a few units per sum
             got, want = out[i, ~own, 0], ref[~own]
             assert T.isfinite(got).all() and ((got - want).norm() / want.norm()).item() < 1e-5
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("q_h,k_h,v_h,d", [(12, 2, 2, 128), (12, 1, 2, 128), (15, 1, 5, 64), (12, 1, 3, 128)])
+@pytest.mark.parametrize("L,gap", [(33, 12.0), (4096, 17.0), (4096, 28.0), (20000, 40.0)])
+def test_dense_dominating_keys(dt, q_h, k_h, v_h, d, L, gap):
+    """Keys `gap` nats above the rest (in every wave's range) whose values are 0, as attention sinks have: the output is
+    what the small weights give, in either type held to 24 bits."""
+    import torch as T
+    b = 8
+    g = T.Generator(device="cuda").manual_seed(L + q_h)
+    tdt = T.bfloat16 if dt == "bf16" else T.float16
+    q, k, v = (T.randn(b, h, n, d, generator=g, device="cuda") for h, n in ((q_h, 1), (k_h, L), (v_h, L)))
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[:, :, ::32] = 0.0
+    k[:, :, ::32, 0] = gap * d ** 0.5 / 8.0
+    v += 0.5
+    v[:, :, ::32] = 0.0
+    q, k, v = q.to(tdt), k.to(tdt), v.to(tdt)
+    out = ops.dense_decode(q, k, v, out_dtype=T.float32).double()
+    for i in range(b):
+        kk, vv = k[i].double().repeat_interleave(q_h // k_h, 0), v[i].double().repeat_interleave(q_h // v_h, 0)
+        ref = (T.softmax((q[i].double() @ kk.transpose(1, 2)) / d ** 0.5, -1) @ vv)[:, 0]
+        # logits of up to 40 rounded to fp32 and exp of them: 40 * 2^-23 = 5e-6 per weight
+        assert ((out[i, :, 0] - ref).norm() / ref.norm()).item() < 1e-5
