@@ -39,7 +39,8 @@ def test_rmsnorm_rows(dt, N, H):
 
 
 @pytest.mark.parametrize("dt", DTS)
-@pytest.mark.parametrize("N,H", [(1, 8), (3, 24), (7, 2560), (2, 8960), (65, 1016), (3, 1004)])
+@pytest.mark.parametrize("N,H", [(1, 8), (3, 24), (7, 2560), (2, 8960), (65, 1016), (3, 1004), (75000, 8), (25003, 24),
+                                 (235, 2560), (67, 8960), (591, 1016), (599, 1004), (1, 600008)])
 def test_silu_mul_rows(dt, N, H):
     g = torch.Generator(device="cuda").manual_seed(N + H)
     x = (torch.randn(N, 2 * H, generator=g, device="cuda") * 3).to(dt)
@@ -58,8 +59,18 @@ def test_silu_mul_extremes():
     vals = [0.0, -0.0, 90.0, -90.0, big, -big, float("inf"), -float("inf"), float("nan"), 1.0]
     g = torch.tensor([v for v in vals for _ in vals] + [0.0] * 4, device="cuda").bfloat16()
     u = torch.tensor(vals * len(vals) + [0.0] * 4, device="cuda").bfloat16()
-    x = torch.cat([g, u]).reshape(1, -1)
+    x = torch.cat([g, u]).reshape(1, -1).repeat(6000, 1)  # the vector form's sizes
     torch.testing.assert_close(ops.silu_mul(x), ops.silu_mul(_unaligned(x)), rtol=0, atol=0, equal_nan=True)
+    torch.testing.assert_close(ops.silu_mul(x)[:1], ops.silu_mul(x[:1]), rtol=0, atol=0, equal_nan=True)
+
+
+def test_silu_mul_past_the_threads_of_a_launch():
+    """2^35 and more outputs, all of one value, in rows 8 elements apart: only the last thread writes the last ones."""
+    N, H = 65535, (1 << 19) + 2048
+    x = torch.full((1, 2 * H), 1.5, device="cuda", dtype=torch.bfloat16)
+    y = torch.zeros(8 * (N - 1) + H, device="cuda", dtype=torch.bfloat16)
+    ops.silu_mul(x.expand(N, -1), out=y.as_strided((N, H), (8, 1)))
+    assert bool((y == ops.silu_mul(x)[0, 0]).all())
 
 
 @pytest.mark.parametrize("dt", DTS)
