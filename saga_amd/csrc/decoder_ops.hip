@@ -27,19 +27,17 @@ __device__ __forceinline__ u32x4 pack16(const float (&f)[8]) {
 }
 
 // A prompt's rotation + append, 16-bit types with 16-byte aligned rows (the
-// kernel below takes every other call).  A block computes the cos / sin of
-// its kRopeTok tokens once, in LDS, and applies them to all of their heads in
-// 16-byte vectors: bound by the bytes of the projection (read once, written
-// once).  One 64-lane block per (token, head) recomputed the same powf and
-// sincosf for every head and moved 2 bytes per lane: 4001 tokens of 15 heads,
-// d 128 (31 MB) 25.4 us, here 9.9.
-constexpr int kRopeTok = 4;
-
+// kernel below takes every other call, and few tokens).  A block computes the
+// cos / sin of its tokens (1 or 2) once, in LDS, and applies them to all of
+// their heads in 16-byte vectors: bound by the bytes of the projection (read
+// once, written once).  One 64-lane block per (token, head) recomputed the
+// same powf and sincosf for every head and moved 2 bytes per lane: 4001 tokens
+// of 15 heads, d 128 (31 MB) 23.4 us, here 9.2.
 template <int DT>
-__global__ void __launch_bounds__(256) rope_kv_append_vec_kernel(RopeParams p) {
-  extern __shared__ float rot[];  // [kRopeTok][2][d / 2]: cos, sin
+__global__ void __launch_bounds__(256) rope_kv_append_vec_kernel(RopeParams p, int tokens) {
+  extern __shared__ float rot[];  // [tokens][2][d / 2]: cos, sin
   const int half = p.d / 2, nh = half / 8, nv = p.d / 8;
-  const int t0 = blockIdx.x * kRopeTok, nt = min(kRopeTok, p.N - t0);
+  const int t0 = blockIdx.x * tokens, nt = min(tokens, p.N - t0);
   for (int e = threadIdx.x; e < nt * half; e += 256) {
     const int t = e / half, i = e - t * half;
     float cs, sn;
@@ -139,13 +137,19 @@ static bool rope_vec(const RopeParams& p) {
 }
 
 hipError_t launch_rope_kv_append(const RopeParams& p, hipStream_t st) {
-  if (rope_vec(p)) {
-    const dim3 grid((p.N + kRopeTok - 1) / kRopeTok);
-    const size_t lds = sizeof(float) * kRopeTok * p.d;
+  // Measured (us; heads q + k + v): element form, 1, 2, 4 tokens per block.  15 heads, d 128: 64 tokens 3.0, 3.5, 3.8,
+  // 4.9; 128 3.4, 3.5, 3.8, 4.9; 256 4.0, 3.6, 3.9, 5.0; 1024 7.7, 4.2, 4.7, 5.4; 2048 12.8, 6.2, 5.8, 6.5; 4001 23.4,
+  // 10.6, 9.2, 9.3.  21 heads, d 64: 128 3.4, 3.4, 3.6, 4.7; 4001 28.7, 8.4, 7.9, 7.6.  (The element form's blocks are
+  // its tokens times heads; at 2^25 tokens a launch of 2 per block ends.)
+  const int64_t blocks = static_cast<int64_t>(p.N) * (p.n_q + p.n_k + p.n_v);
+  if (rope_vec(p) && blocks >= 3072 && p.N < (1 << 25)) {
+    const int tokens = p.N < 1536 ? 1 : 2;
+    const dim3 grid((p.N + tokens - 1) / tokens);
+    const size_t lds = sizeof(float) * tokens * p.d;
     if (p.dt == SAGA_DTYPE_BF16)
-      hipLaunchKernelGGL((rope_kv_append_vec_kernel<SAGA_DTYPE_BF16>), grid, dim3(256), lds, st, p);
+      hipLaunchKernelGGL((rope_kv_append_vec_kernel<SAGA_DTYPE_BF16>), grid, dim3(256), lds, st, p, tokens);
     else
-      hipLaunchKernelGGL((rope_kv_append_vec_kernel<SAGA_DTYPE_F16>), grid, dim3(256), lds, st, p);
+      hipLaunchKernelGGL((rope_kv_append_vec_kernel<SAGA_DTYPE_F16>), grid, dim3(256), lds, st, p, tokens);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(rope_kv_append_kernel, dim3(p.N, p.n_q + p.n_k + p.n_v), dim3(64), 0, st, p);

@@ -75,10 +75,13 @@ def test_silu_mul_past_the_threads_of_a_launch():
 
 @pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("N,n_q,n_k,n_v,d", [(1, 12, 1, 2, 128), (4, 15, 1, 5, 64), (5, 3, 1, 1, 16), (67, 12, 2, 2, 128),
-                                             (6, 4, 2, 4, 48), (5, 2, 1, 1, 24)])
+                                             (6, 4, 2, 4, 48), (5, 2, 1, 1, 24),
+                                             # 3072 (token, head) pairs and more: vectors, 1 token per block, 2 from 1536
+                                             (205, 12, 1, 2, 128), (147, 15, 1, 5, 64), (613, 3, 1, 1, 16), (310, 4, 2, 4, 48),
+                                             (1535, 3, 1, 1, 16), (1537, 12, 1, 2, 128), (1601, 2, 1, 1, 24)])
 def test_rope_kv_append_rows(dt, N, n_q, n_k, n_v, d):
     g = torch.Generator(device="cuda").manual_seed(N + d)
-    B, Lmax = 3, 80
+    B, Lmax = 3, max(80, N)
     qkv = torch.randn(N, (n_q + n_k + n_v) * d, generator=g, device="cuda").to(dt)
     pos = torch.randperm(Lmax, generator=g, device="cuda")[:N].int()
     pos[N // 2] = Lmax if N > 4 else pos[N // 2]  # out of range: NaN queries, no cache row
