@@ -1079,7 +1079,9 @@ int saga_prefill_attention(const saga_tensor* query, const saga_tensor* key, con
     return fail(SAGA_ERR_INVALID, "prefill: causal_offset out of range");
   if (!(scale > 0.f) || !std::isfinite(scale))
     return fail(SAGA_ERR_UNSUPPORTED, "prefill: scale must be positive and finite");
-  const int64_t nmb = prefill_query_blocks(b, q_h, Lq, Lk, static_cast<int>(d), mask != nullptr);
+  const int64_t keys = causal ? std::max<int64_t>(std::min<int64_t>(Lk, Lq + causal_offset), 0) : Lk;
+  const PrefillShape shape = prefill_shape(b, q_h, Lq, keys, static_cast<int>(d), mask != nullptr);
+  const int64_t nmb = prefill_query_blocks(shape, Lq);
   if (nmb * q_h * b >= (1LL << 31)) return fail(SAGA_ERR_UNSUPPORTED, "prefill: grid too large");
   if ((rc = check_vec_rows(query, "query")) || (rc = check_vec_rows(key, "key")) || (rc = check_vec_rows(value, "value")))
     return rc;
@@ -1127,6 +1129,7 @@ int saga_prefill_attention(const saga_tensor* query, const saga_tensor* key, con
   p.Lq = static_cast<int32_t>(Lq);
   p.Lk = static_cast<int32_t>(Lk);
   p.nmb = static_cast<int32_t>(nmb);
+  p.shape = shape;
   p.causal = causal ? 1 : 0;
   p.causal_off = static_cast<int32_t>(causal_offset);
   p.scale = scale;

@@ -296,6 +296,11 @@ hipError_t launch_prompt_mlp(const PromptMlpParams& p, hipStream_t st);
 // Prefill attention with separate key / value head maps (csrc/prefill.hip).
 // Strides in elements; q [b, q_h, Lq, d], k [b, k_h, Lk, d], v [b, v_h, Lk, d],
 // mask [b|1, q_h|1, Lq, Lk] (broadcast dims stride 0), out [b, Lq, q_h, d].
+// Waves per block and wave groups that split the keys (32 * nw / ks queries
+// per block).
+struct PrefillShape {
+  int32_t nw, ks;
+};
 struct PrefillParams {
   const char* q;
   int64_t q_sb, q_sh, q_sl;
@@ -310,17 +315,13 @@ struct PrefillParams {
   int64_t o_sb, o_sq, o_sh;
   int32_t b, q_h, k_h, v_h, Lq, Lk;
   int32_t nmb;         // query blocks per (batch, head)
+  PrefillShape shape;
   int32_t causal;      // key j visible to query i iff j <= i + causal_off
   int32_t causal_off;
   float scale;
 };
-// Waves per block, wave groups that split the keys (32 * nw / ks queries per
-// block), and query blocks per (batch, head).
-struct PrefillShape {
-  int nw, ks;
-};
-PrefillShape prefill_shape(int64_t b, int64_t q_h, int64_t Lq, int64_t Lk, int d, bool masked);
-int64_t prefill_query_blocks(int64_t b, int64_t q_h, int64_t Lq, int64_t Lk, int d, bool masked);
+PrefillShape prefill_shape(int64_t b, int64_t q_h, int64_t Lq, int64_t keys, int d, bool masked);
+int64_t prefill_query_blocks(const PrefillShape& shape, int64_t Lq);
 hipError_t launch_prefill_attention(int dtype, int d, const PrefillParams& p, hipStream_t st);
 
 }  // namespace saga

@@ -199,15 +199,16 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
     load_rows(kb, krow, st * S::BNS, kr);
     load_rows(vb, vrow, (st - 1) * S::BNS, vr);
   };
-  // V rows of stage st at or past Lk are copies of the last row: their weight
-  // is 0, but 0 * inf is NaN, so zeros are staged in their place.  No stage
-  // that load_stage_full loads has such rows.
+  // V rows at or past Lk are copies of the last row: their weight is 0, but 0 *
+  // inf is NaN, so zeros are staged in their place.  One stage has such rows
+  // beside others, and load_stage_full never loads it.  (Tested ahead of the
+  // matrix phase: a branch between its MFMAs and the staging keeps them apart.)
+  const int tail = p.Lk % S::BNS ? p.Lk / S::BNS + 1 : -1;
   auto zero_tail = [&](int st) {
-    const int r0 = (st - 1) * S::BNS;
-    if (r0 + S::BNS <= p.Lk) return;
+    if (st != tail) return;
 #pragma unroll
     for (int i = 0; i < S::KPT; ++i)
-      if (r0 + lr + i * S::RPP >= p.Lk) vr[i] = u32x4{0u, 0u, 0u, 0u};
+      if ((st - 1) * S::BNS + lr + i * S::RPP >= p.Lk) vr[i] = u32x4{0u, 0u, 0u, 0u};
   };
   // the next stage of a run of stages whose K rows lie below Lk, near
   const char* kcur = kb + 3 * S::BNS * krow + koffs;
@@ -456,8 +457,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
     lds_sync();
     if (second) lds_sync();  // the second half runs one phase behind the first; a barrier ends every phase
     bool vis = nmine > 0 && mask_visible();
-    if (vis) qk(0);
     zero_tail(1);
+    if (vis) qk(0);
     write_stage(1);
     load_stage(2);
     if constexpr (kPing) lds_sync();
@@ -475,10 +476,10 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
       if (vis) softmax(it);
       load_mask(it + 1);
       lds_sync();
+      zero_tail(it + 2);
       if (vis) pv(it + 1);
       const bool next = it + 1 < nmine && mask_visible();
       if (next) qk(it + 1);
-      zero_tail(it + 2);
       write_stage(it + 2);
       load_stage(it + 3);
       vis = next;
@@ -533,7 +534,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(PrefillParams 
 }
 
 template <int DT, int D>
-void launch_prefill_shape(const PrefillParams& p, PrefillShape sh, dim3 grid, hipStream_t st) {
+void launch_prefill_shape(const PrefillParams& p, dim3 grid, hipStream_t st) {
+  const PrefillShape sh = p.shape;
   if (!p.mask) {
     if (sh.nw == 4) hipLaunchKernelGGL((prefill_attn_kernel<DT, D, 4, 1, kPfNone>), grid, dim3(256), 0, st, p);
     else if (sh.ks == 2) hipLaunchKernelGGL((prefill_attn_kernel<DT, D, 8, 2, kPfNone>), grid, dim3(512), 0, st, p);
@@ -552,36 +554,38 @@ template <int DT>
 hipError_t launch_prefill_typed(int d, const PrefillParams& p, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(p.nmb) * static_cast<unsigned>(p.q_h * p.b));
   if (grid.x == 0) return hipSuccess;
-  const PrefillShape sh = prefill_shape(p.b, p.q_h, p.Lq, p.Lk, d, p.mask != nullptr);
-  if (d == 128) launch_prefill_shape<DT, 128>(p, sh, grid, st);
-  else launch_prefill_shape<DT, 64>(p, sh, grid, st);
+  if (d == 128) launch_prefill_shape<DT, 128>(p, grid, st);
+  else launch_prefill_shape<DT, 64>(p, grid, st);
   return hipGetLastError();
 }
 
 }  // namespace
 
-// Waves per block and key split.  A launch of at most one block of 256
-// queries per CU is bound by its longest chain of tiles: the block's waves
-// split the keys (4 waves over 128 queries, two tiles per stage; 4001 tokens of
-// 12 heads, d 128: 73 us against 95 with 4 unsplit waves and 101 with 8), unless
-// that takes a second round of blocks for a short chain (8 x 512 tokens: 27
-// against 22 us).  Larger launches: 8 waves from 8192 keys at d 128 (32768
+// Waves per block and key split, by the keys that the last query can see.  A
+// launch of at most one block of 256 queries per CU is bound by its longest
+// chain of tiles: the block's waves split the keys (4 waves over 128 queries,
+// two tiles per stage; 4001 tokens of 12 heads, d 128: 73 us against 95 with 4
+// unsplit waves and 101 with 8), unless that takes a second round of blocks
+// for a short chain (8 x 512 tokens: 27 against 22 us), or the chain is so
+// short that its start and the merge count for more (12 heads, d 128, split
+// against 4 waves: 64 tokens 8.4 and 6.1 us, 256 12.5 and 11.5, 384 14.8 and
+// 13.9, 512 16.5 and 16.3, 700 18.0 and 18.6; d 64, 15 heads: 64 6.2 and 4.8, 320
+// 8.9 and 8.7, 384 9.8 and 10.2).  Larger launches: 8 waves from 8192 keys at d 128 (32768
 // tokens: 2.9 ms against 3.2 with 4), else 4 (d 64, 32768 tokens: 2.14 against
 // 2.19 ms).  Masked: always 4 (2999 tokens, boolean mask: 125 us against 143
 // split and 171 with 8; now 103), whose waves skip the tiles that the mask hides.
-PrefillShape prefill_shape(int64_t b, int64_t q_h, int64_t Lq, int64_t Lk, int d, bool masked) {
+PrefillShape prefill_shape(int64_t b, int64_t q_h, int64_t Lq, int64_t keys, int d, bool masked) {
   constexpr int64_t kCUs = 256;
   if (masked) return {4, 1};
   const int64_t units = b * q_h;
   if ((Lq + 255) / 256 * units <= kCUs) {
-    if ((Lq + 127) / 128 * units <= kCUs || Lk >= 1536) return {8, 2};
+    if (keys > (d == 128 ? 384 : 320) && ((Lq + 127) / 128 * units <= kCUs || keys >= 1536)) return {8, 2};
     return {4, 1};
   }
-  return d == 128 && Lk >= 8192 ? PrefillShape{8, 1} : PrefillShape{4, 1};
+  return d == 128 && keys >= 8192 ? PrefillShape{8, 1} : PrefillShape{4, 1};
 }
 
-int64_t prefill_query_blocks(int64_t b, int64_t q_h, int64_t Lq, int64_t Lk, int d, bool masked) {
-  const PrefillShape sh = prefill_shape(b, q_h, Lq, Lk, d, masked);
+int64_t prefill_query_blocks(const PrefillShape& sh, int64_t Lq) {
   const int64_t bm = 32 * sh.nw / sh.ks;
   return (Lq + bm - 1) / bm;
 }

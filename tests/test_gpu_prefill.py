@@ -201,7 +201,10 @@ def _ref64(q, k, v, rows, causal, off, mask=None):
     (1, 12, 1, 2, 128, 127, 129, True, 2), (1, 12, 1, 2, 128, 1537, 1537, True, 0), (2, 15, 1, 5, 64, 1600, 1600, True, 0),
     (1, 12, 1, 2, 128, 70, 3011, False, 0), (1, 4, 1, 1, 64, 300, 1000, True, 700), (1, 4, 1, 1, 128, 300, 200, True, -150),
     (8, 12, 1, 2, 128, 321, 321, True, 0), (8, 15, 1, 5, 64, 200, 257, False, 0), (3, 24, 2, 2, 128, 1100, 1100, True, 0),
-    (1, 12, 1, 2, 128, 8200, 8200, True, 0), (1, 16, 1, 1, 128, 4200, 8255, False, 0), (1, 15, 1, 5, 64, 8193, 8193, True, 0)])
+    # up to 320 (d 64) and 384 visible keys unsplit, then split; split stages that end inside either wave group's tile
+    (1, 4, 2, 1, 64, 320, 320, True, 0), (1, 4, 2, 1, 64, 321, 321, True, 0), (1, 4, 2, 1, 128, 385, 385, True, 0), (1, 4, 1, 2, 128, 33, 449, False, 0),
+    (1, 4, 1, 1, 128, 129, 511, False, 0), (1, 4, 1, 1, 64, 70, 513, False, 0), (1, 4, 1, 2, 128, 128, 900, True, 256),
+    (1, 4, 1, 2, 128, 128, 900, True, 257), (1, 12, 1, 2, 128, 8200, 8200, True, 0), (1, 16, 1, 1, 128, 4200, 8255, False, 0), (1, 15, 1, 5, 64, 8193, 8193, True, 0)])
 def test_prefill_block_shapes(b, q_h, k_h, v_h, d, Lq, Lk, causal, off):
     g = torch.Generator(device="cuda").manual_seed(Lq + Lk)
     q = torch.randn(b, Lq, q_h, d, generator=g, device="cuda").bfloat16().transpose(1, 2)
@@ -260,7 +263,8 @@ def test_prefill_far_rows():
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", ["full", "causal", "bool", "half", "float"])
 @pytest.mark.parametrize("b,q_h,Lq,Lk,d", [(1, 4, 70, 65, 64), (1, 4, 70, 65, 128), (2, 4, 33, 129, 64), (1, 4, 130, 129, 128),
-                                           (1, 4, 70, 128, 128), (11, 12, 130, 129, 64), (11, 12, 130, 65, 128),
+                                           (1, 4, 70, 128, 128), (1, 4, 70, 385, 128), (2, 4, 33, 449, 64),
+                                           (1, 4, 130, 513, 128), (1, 4, 70, 512, 128), (11, 12, 130, 129, 64), (11, 12, 130, 65, 128),
                                            (22, 12, 1, 8193, 128)])
 def test_prefill_infinite_last_value(b, q_h, Lq, Lk, d, kind, dt):
     """An infinite value in the last key row makes that dim infinite for the queries that see the row: what a partial
