@@ -221,7 +221,7 @@ def test_prefill_block_shapes(b, q_h, k_h, v_h, d, Lq, Lk, causal, off):
     assert torch.isfinite(out).all() and ((out - ref).norm() / ref.norm().clamp(min=1e-9)).item() < 5e-3
 
 
-@pytest.mark.parametrize("kind", ["bool", "bytes", "half", "float", "strided"])
+@pytest.mark.parametrize("kind", ["bool", "bytes", "half", "float", "strided", "strided half", "strided float"])
 @pytest.mark.parametrize("b,h,d,Lq,Lk", [(2, 4, 64, 130, 191), (1, 2, 128, 257, 257), (3, 3, 128, 33, 64), (2, 2, 64, 5, 7)])
 def test_prefill_mask_loads(kind, b, h, d, Lq, Lk):
     """Each way a mask reaches the kernel, rows at odd addresses, tiles wholly hidden, wholly visible and mixed,
@@ -236,13 +236,13 @@ def test_prefill_mask_loads(kind, b, h, d, Lq, Lk):
     mask = keep
     if kind == "bytes":  # any non-zero byte keeps, as a cast to bool does
         mask = (keep.to(torch.uint8) * 5).view(torch.bool)
-    elif kind in ("half", "float"):
+    elif kind.endswith(("half", "float")):
         mask = torch.randn(keep.shape, generator=g, device="cuda").masked_fill(~keep, float("-inf"))
-        mask = mask.to(torch.bfloat16 if kind == "half" else torch.float32)
-    elif kind == "strided":
-        mask = keep.transpose(2, 3).contiguous().transpose(2, 3)
+        mask = mask.to(torch.bfloat16 if kind.endswith("half") else torch.float32)
+    if kind.startswith("strided"):
+        mask = mask.transpose(2, 3).contiguous().transpose(2, 3)
     got = ops.prefill_attention(q, k, v, mask).double()
-    ref = _ref64(q, k, v, torch.arange(Lq, device="cuda"), False, 0, mask if kind in ("half", "float") else keep)
+    ref = _ref64(q, k, v, torch.arange(Lq, device="cuda"), False, 0, keep if mask.dtype == torch.bool else mask)
     assert ((got - ref).norm() / ref.norm()).item() < 5e-3 and not got[:, Lq // 3].any()
 
 
