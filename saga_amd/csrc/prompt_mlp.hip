@@ -144,7 +144,12 @@ __device__ __forceinline__ void mlp_block(const PromptMlpParams& p, int t0, int 
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const float g = acc[i][j][2 * q], u = acc[i][j][2 * q + 1];
-        o[q] = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
+        // The hardware's reciprocal flushes results below 2^-126 (gates from -87.3
+        // down to -88.7, where exp overflows): taken in 2^-32 units.  With the
+        // hardware's exp the activation is within 8e-6 of exact before its
+        // rounding to bf16; expf and a division cost 10 % of the kernel (4001
+        // tokens, 17920 x 1536: 201 -> 220 us).
+        o[q] = g * (__builtin_amdgcn_rcpf((1.0f + __expf(-g)) * 0x1p-32f) * 0x1p-32f) * u;
       }
       const uint32_t bits = f32_to_bf16_bits(o[0]) | (static_cast<uint32_t>(f32_to_bf16_bits(o[1])) << 16);
       *reinterpret_cast<uint32_t*>(lds + (16 * (wm * MF + i) + col) * OROW + (wn * NF + j) * 16 + s * 4) = bits;

@@ -47,6 +47,22 @@ def test_prompt_mlp_special_values():
     assert bool(y[2].isnan().all()) and bool((y[3:] == 0).all())
 
 
+def test_prompt_mlp_vanishing_gates():
+    """silu where 1 / (1 + exp(-gate)) is a subnormal number (gates of -87.4 to -88.7) and around."""
+    K, N = 64, 32
+    gates = torch.cat([torch.arange(-89.0, -80.0, 0.5), torch.arange(-80.0, 20.0, 1.0)]).cuda()
+    x = torch.zeros(len(gates), K, device="cuda", dtype=torch.bfloat16)
+    x[:, 0], x[:, 1] = gates, 1.0
+    w = torch.zeros(N, K, device="cuda", dtype=torch.bfloat16)
+    w[0::2, 0], w[1::2, 1] = 1.0, 2.0 ** 100
+    y = ops.prompt_mlp(x, ops.pack_gemv_weight(w)).double()
+    g = gates.bfloat16().double()
+    want = (g * torch.sigmoid(g) * 2.0 ** 100)[:, None]
+    # one rounding to bf16 (2^-8 at most) and the fp32 activation's 8e-6; below -88.7 exp overflows and silu is 0
+    fine = (g > -88.7)[:, None]
+    assert bool((((y - want).abs() <= want.abs() * (2.0 ** -8 + 1e-5)) | ~fine).all())
+
+
 def test_prompt_mlp_refuses():
     x = torch.zeros(4, 96, device="cuda", dtype=torch.bfloat16)
     w = ops.pack_gemv_weight(torch.zeros(32, 96, device="cuda", dtype=torch.bfloat16))
