@@ -1010,9 +1010,10 @@ int saga_prompt_mlp(const saga_tensor* x, const saga_tensor* w, saga_tensor* y, 
   if ((rc = check_packed(w, K))) return rc;
   if (y->shape[0] != T || y->shape[1] != N / 2) return fail(SAGA_ERR_INVALID, "prompt_mlp: y must be [T, N / 2]");
   if (K % 64 || K >= (1LL << 24)) return fail(SAGA_ERR_UNSUPPORTED, "prompt_mlp: K %% 64 == 0 required");
-  if (T >= (1LL << 24) || N >= (1LL << 24)) return fail(SAGA_ERR_UNSUPPORTED, "prompt_mlp: sizes too large");
+  // at most two blocks per 256 x 256 outputs, and a launch holds less than 2^32 threads
+  if (T >= (1LL << 24) || N >= (1LL << 24) || (T + 255) / 256 * ((N + 255) / 256) >= (1LL << 22))
+    return fail(SAGA_ERR_UNSUPPORTED, "prompt_mlp: sizes too large");
   if ((rc = check_vec_rows(x, "x")) || (rc = check_vec_rows(y, "y"))) return rc;
-  if (T == 0 || N == 0 || K == 0) return T && N ? fail(SAGA_ERR_INVALID, "prompt_mlp: K must be positive") : ok();
   PromptMlpParams p{};
   p.x = x->data;
   p.w = w->data;

@@ -268,6 +268,20 @@ def test_pack_gemv_weight_8_row_tiles_on_cpu():
         ops.pack_gemv_weight(torch.zeros(16, 96), 8)
 
 
+def test_prompt_mlp_refuses_more_blocks_than_a_launch_holds():
+    """Rows that share memory (stride 0) reach block counts past 2^31; an empty weight does not exist."""
+    lib = _lib.load()
+
+    def call(T, tiles):
+        x, w = _t((T, 64), strides=(0, 1)), _t((tiles, 2, 16, 32))
+        y = _t((T, tiles * 8), strides=(0, 1))
+        return lib.saga_prompt_mlp(ctypes.byref(x), ctypes.byref(w), ctypes.byref(y), None)
+
+    assert call((1 << 24) - 1, (1 << 20) - 1) == -2 and "too large" in _err()
+    assert call(1 << 20, 1 << 14) == -2 and "too large" in _err()
+    assert call(0, 4) == -1 and call(4, 0) == -1
+
+
 def test_embed_rope_and_advance_argument_errors():
     """The step's opening and close check their operands before any launch."""
     lib = _lib.load()
