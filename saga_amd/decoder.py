@@ -271,19 +271,6 @@ class SagaDecoder:
             self.ws["gemv"] = buf(max(lib.saga_gemv_workspace_bytes(B, n, k) for n, k in shapes))
             self.ws["argmax"] = buf(lib.saga_argmax_workspace_bytes(B, s.vocab))
 
-    @staticmethod
-    def _unpack(w: torch.Tensor) -> torch.Tensor:
-        """Row-major [N, K] of a packed weight: [N/16, K/32, 16, 32] or, in
-        8-row tiles, [N/8, K/64, 512], in torch (any device; the prefill uses
-        ops.unpack_gemv_weights)."""
-        if w.dim() == 2:
-            return w
-        if w.dim() == 3:
-            n8, k64 = w.shape[0], w.shape[1]
-            return w.reshape(n8, k64, 2, 8, 32).permute(0, 3, 1, 2, 4).reshape(n8 * 8, k64 * 64)
-        n16, k32 = w.shape[0], w.shape[1]
-        return w.permute(0, 2, 1, 3).reshape(n16 * 16, k32 * 32)
-
     def _prefill_layer(self, l: int):
         """(norm-1 weight, w_qkv, w_o, norm-2 weight, w_gu, w_d), row-major and
         in natural row order, for the prefill of layer l: the originals, or,

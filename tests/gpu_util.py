@@ -41,3 +41,13 @@ def qkv(rng, b, q_h, k_h, v_h, d, L, dt, qscale=1.0, outliers=0.0):
     k = round_to(kf, dt)
     v, vd = randn(rng, (b, v_h, L, d), dt)
     return (q, k, v), (qd, dev(k, dt), vd)
+
+
+def unpack_rows(w: torch.Tensor) -> torch.Tensor:
+    """Row-major [N, K] of a packed weight, [N/16, K/32, 16, 32] or, in 8-row tiles, [N/8, K/64, 512]
+    (ops.pack_gemv_weight), by torch's permutes."""
+    if w.dim() == 3:
+        n8, k64 = w.shape[0], w.shape[1]
+        return w.reshape(n8, k64, 2, 8, 32).permute(0, 3, 1, 2, 4).reshape(n8 * 8, k64 * 64)
+    n16, k32 = w.shape[0], w.shape[1]
+    return w.permute(0, 2, 1, 3).reshape(n16 * 16, k32 * 32)

@@ -253,17 +253,17 @@ def test_gemv_packed8_weight_layout_checks():
 
 def test_pack_gemv_weight_8_row_tiles_on_cpu():
     """pack_gemv_weight(w, 8)[t, j, 32 r + c] = w[8t + r % 8, 64j + 32 (r // 8) + c],
-    and the decoder's unpacking inverts both layouts."""
+    and the tests' unpacking inverts both layouts."""
     import torch
+    from gpu_util import unpack_rows
     from saga_amd import ops
-    from saga_amd.decoder import SagaDecoder
     w = torch.arange(32 * 192, dtype=torch.float32).reshape(32, 192)
     p = ops.pack_gemv_weight(w, 8)
     assert p.shape == (4, 3, 512)
     for t, j, r, c in [(0, 0, 0, 0), (3, 2, 15, 31), (1, 1, 8, 5), (2, 0, 7, 30)]:
         assert p[t, j, 32 * r + c] == w[8 * t + r % 8, 64 * j + 32 * (r // 8) + c]
     for rows in (16, 8):
-        assert torch.equal(SagaDecoder._unpack(ops.pack_gemv_weight(w, rows)), w)
+        assert torch.equal(unpack_rows(ops.pack_gemv_weight(w, rows)), w)
     with pytest.raises(ValueError, match="K % 64"):
         ops.pack_gemv_weight(torch.zeros(16, 96), 8)
 

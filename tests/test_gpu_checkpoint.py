@@ -76,3 +76,28 @@ def test_generate_graphs_equal_eager_steps(tmp_path):
     top2 = np.sort(ref)[-2:]
     if top2[1] - top2[0] > 0.05:
         assert int(g[0, 0]) == int(np.argmax(ref))
+
+
+@pytest.mark.parametrize("kind,tie,keep,vocab", [("qwen2", True, False, 1024), ("qwen2", True, True, 1024), ("llama", False, False, 1024),
+                                                 ("llama", False, True, 1024), ("qwen2", True, False, 1000)])
+def test_prompt_first_token(tmp_path, kind, tie, keep, vocab):
+    """The token a prompt leaves, through each LM head that a decoder may hold for it (tied or its own row-major weight, the
+    packed copy, a vocabulary that the 16-row kernel does not take), is the float64 forward's for prompts whose margin is
+    clear."""
+    from saga_amd.checkpoint import load_checkpoint
+    from saga_amd.decoder import SagaDecoder
+    model = tiny_hf_model(kind, n_kv=2, n_k_shared=1, tie=tie, d=64, intermediate=512, vocab=vocab)
+    path = str(tmp_path / "saga")
+    save_saga_checkpoint(model, path, n_k=1)
+    m = SagaDecoder.from_pretrained(path, batch=2, max_len=128, keep_source_weights=keep)
+    shape, w = load_checkpoint(path)
+    rng, clear = np.random.default_rng(11), 0
+    for _ in range(8):
+        ids = [int(t) for t in rng.integers(0, vocab, int(rng.integers(1, 100)))]
+        m.prefill(torch.tensor(ids))
+        ref = forward64(shape, w, ids)[-1]
+        top2 = np.sort(ref)[-2:]
+        if top2[1] - top2[0] > 0.05:
+            clear += 1
+            assert m.tokens.tolist() == [int(np.argmax(ref))] * 2
+    assert clear >= 2

@@ -153,3 +153,66 @@ def test_dense_dominating_keys(dt, q_h, k_h, v_h, d, L, gap):
         ref = (T.softmax((q[i].double() @ kk.transpose(1, 2)) / d ** 0.5, -1) @ vv)[:, 0]
         # logits of up to 40 rounded to fp32 and exp of them: 40 * 2^-23 = 5e-6 per weight
         assert ((out[i, :, 0] - ref).norm() / ref.norm()).item() < 1e-5
+
+
+LAYOUTS = [(4, 12, 2, 2, 128), (4, 12, 1, 2, 128), (4, 8, 2, 1, 128), (5, 15, 1, 5, 64), (4, 16, 4, 8, 64), (2, 16, 1, 1, 64),
+           (4, 12, 1, 3, 128), (4, 16, 1, 4, 64)]
+
+
+def _dense64(q, k, v, x_add):
+    """float64 attention of one batch row: q [q_h, 1, d], k / v [h, n, d], x_add [1 or q_h, n] added to the logits."""
+    q_h, _, d = q.shape
+    kk, vv = (t.double().repeat_interleave(q_h // t.shape[0], 0) for t in (k, v))
+    x = (q.double() @ kk.transpose(1, 2))[:, 0] / d ** 0.5 + x_add
+    return (torch.softmax(x, -1)[:, None] @ vv)[:, 0]
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mask", [None, "bool", "float", "heads"])
+@pytest.mark.parametrize("b,q_h,k_h,v_h,d", LAYOUTS)
+@pytest.mark.parametrize("L", [1, 33, 1055])
+def test_dense_value_head_layouts_numeric(dt, mask, b, q_h, k_h, v_h, d, L):
+    """Every head of every layout against 64 bits, with ragged kv_len and with masks (bool adds 1, as the reference does;
+    float broadcast or per head, with -inf)."""
+    g = torch.Generator(device="cuda").manual_seed(L + q_h + d)
+    q, k, v = (torch.randn(b, h, n, d, generator=g, device="cuda").to(dt) for h, n in ((q_h, 1), (k_h, L), (v_h, L)))
+    lens = [max(1, L - 9 * i) for i in range(b)]
+    m = None
+    if mask == "bool":
+        m = torch.rand(b, 1, 1, L, generator=g, device="cuda") < 0.5
+    elif mask:
+        m = torch.randn(b, q_h if mask == "heads" else 1, 1, L, generator=g, device="cuda")
+        m[torch.rand(m.shape, generator=g, device="cuda") < 0.3] = float("-inf")
+        m[..., 0] = 0.0
+    kv = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out = ops.dense_decode(q, k, v, m, kv_len=kv, out_dtype=torch.float32).double()
+    for i, n in enumerate(lens):
+        add = 0.0 if m is None else m[i, :, 0, :n].double()
+        ref = _dense64(q[i], k[i, :, :n], v[i, :, :n], add)
+        # fp32 scores, exp and sums: a few 2^-24 per term
+        assert ((out[i, :, 0] - ref).norm() / ref.norm()).item() < 1e-5
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,q_h,k_h,v_h,d", [c for c in LAYOUTS if c[3] not in (3, 4)])
+@pytest.mark.parametrize("L", [1, 40, 700])
+def test_dense_special_values(dt, b, q_h, k_h, v_h, d, L):
+    """inf, -inf, both, NaN, and an infinite value of weight 0 (NaN), each in a dim of its own of the last value head; all
+    other dims and heads are compared."""
+    g = torch.Generator(device="cuda").manual_seed(L + q_h)
+    q, k, v = (torch.randn(b, h, n, d, generator=g, device="cuda").to(dt) for h, n in ((q_h, 1), (k_h, L), (v_h, L)))
+    inf = float("inf")
+    v[:, -1, 0, 3], v[:, -1, L // 2, 4], v[:, -1, L - 1, 7] = inf, -inf, float("nan")
+    v[:, -1, 0, 5], v[:, -1, L - 1, 5] = inf, -inf  # one value where L is 1: -inf
+    add = torch.zeros(b, 1, 1, L, device="cuda")
+    if L > 1:
+        add[..., 1] = -inf
+        v[:, -1, 1, 9] = inf
+    out = ops.dense_decode(q, k, v, add, out_dtype=torch.float32).double()
+    for i in range(b):
+        ref = _dense64(q[i], k[i], v[i], add[i, :, 0].double())
+        torch.testing.assert_close(out[i, :, 0], ref, rtol=0, atol=1e-5, equal_nan=True)
+        own = ref[q_h - q_h // v_h:]  # the special values' own query heads, and no others
+        assert (own[:, 3] == inf).all() and (own[:, 4] == -inf).all() and own[:, 7].isnan().all()
+        assert own[:, 5].isnan().all() if L > 1 else (own[:, 5] == -inf).all()
+        assert torch.isfinite(ref[: q_h - q_h // v_h]).all() and (L == 1 or own[:, 9].isnan().all())

@@ -5,8 +5,8 @@ take."""
 import pytest
 import torch
 
+from gpu_util import unpack_rows
 from saga_amd import ops
-from saga_amd.decoder import SagaDecoder
 
 pytestmark = pytest.mark.gpu
 DTS = [torch.bfloat16, torch.float16]
@@ -104,7 +104,7 @@ def test_unpack_gemv_weights(rows, N, K):
     w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
     p = ops.pack_gemv_weight(w, rows)
     plain, pairs = ops.unpack_gemv_weights([p, p], [None, (1, N)])
-    assert torch.equal(plain, w) and torch.equal(plain, SagaDecoder._unpack(p))
+    assert torch.equal(plain, w) and torch.equal(plain, unpack_rows(p))
     assert torch.equal(pairs, torch.cat([w[0::2], w[1::2]]))
 
 
@@ -113,7 +113,7 @@ def test_unpack_rotary_heads_and_errors():
     w = torch.randn((n_q + n_k + n_v) * d, K, device="cuda").bfloat16()
     p = ops.pack_gemv_weight(w[ops.rope_pair_order(n_q, n_k, n_v, d, device="cuda")].contiguous(), 8)
     a, b, c = ops.unpack_gemv_weights([p, w, p], [(n_q + n_k, d), None, None])
-    assert torch.equal(a, w) and b is w and torch.equal(c, SagaDecoder._unpack(p))
+    assert torch.equal(a, w) and b is w and torch.equal(c, unpack_rows(p))
     for heads in ((7, d), (1, d - 1), (1, 80), (-1, d)):
         with pytest.raises(RuntimeError, match="unpack"):
             ops.unpack_gemv_weights([p], [heads])
