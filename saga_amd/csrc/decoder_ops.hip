@@ -367,9 +367,9 @@ hipError_t launch_silu_mul(const RowParams& p, hipStream_t st) {
 // together, the writes of a wave 1 KB of one row.  Rows of a rotated head of
 // head_rows rows go from rotary-pair order [0, d/2, 1, d/2 + 1, ...] to
 // natural order on the way.  Bound by HBM (each weight read and written
-// once): the four of a 1.5B layer, 93.6 MB, in 31 us (6.0 TB/s); as torch
-// permutes (and, in place of the row order, a reordering pass over the
-// prompt's q/k/v and gate/up rows) they took 190 us at 4001 tokens.
+// once): the q/k/v, o and down weights of a 1.5B layer, 76 MB moved, in 16.4 us
+// (4.7 TB/s).  As torch permutes (and, in place of the row order, a reordering
+// pass over the prompt's q/k/v rows) they and gate/up took 190 us at 4001 tokens.
 __global__ void __launch_bounds__(256) unpack_kernel(UnpackParams p) {
   int it = 0;
   while (it + 1 < p.n && static_cast<int>(blockIdx.x) >= p.item[it + 1].block0) ++it;

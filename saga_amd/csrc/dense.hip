@@ -16,8 +16,10 @@
 // Waves merge in LDS; with several splits each writes a (max, sum, o[d])
 // partial per head and kernel 2 (one block per head) merges them.
 //
-// 16-bit caches whose units hold whole value heads (1, 2 or 5 of them) take
-// dense_mfma_kernel instead: both products on MFMA, see there.
+// 16-bit caches whose units hold whole value heads (1, 2 or, at d 64, 5 of
+// them) take dense_mfma_kernel instead: both products on MFMA, see there.  These
+// are the units of the decoder's shapes; it is built and measured for no other
+// count (3, 4, 8; 5 at d 128), which stay here.
 #include <type_traits>
 
 #include "common.cuh"
@@ -316,10 +318,13 @@ struct DenseMfma {
 // (QK, LDS write) and refilled with the next step's before its softmax and
 // second product: the stream does not wait for either.  The VALU kernel
 // above spends 12 FMAs per value element and head group and loads value heads
-// past the second in a dependent burst.  Whole calls: 8 x 33024 positions,
-// 12 / 2 / 2 heads, d 128: 73.2 -> 58.5 us (4.63 TB/s), 12 / 1 / 2 heads 63.4 ->
-// 48.5; 16 x 16384, 15 / 5 / 5 heads, d 64: 129 -> 77; 4 rows of up to 8195, 15 /
-// 1 / 5 heads, d 64: 22.2 -> 16.7 (latency: one block per CU, two launches).
+// past the second in a dependent burst.  Both kernels of a call, 20 calls in one
+// captured graph (on data that the last-level cache partly keeps): 8 x 33024
+// positions, 12 / 2 / 2 heads, d 128: 63.0 -> 47.4 us; 4 x 33024, 12 / 1 / 2
+// heads: 35.0 -> 26.6; d 64, 4 x 33024: 15 / 1 / 5 heads 41.5 -> 33.0, 15 / 5 / 5
+// heads 62.1 -> 36.8; 4 x 4096, 15 / 1 / 5 heads: 13.0 -> 10.3 (latency: one block
+// per CU, two launches).  f16 the same within 4 %, and up to a third more where
+// logits 30 nats apart need further terms.
 template <int DT, int D, int NV>
 __global__ void __launch_bounds__(256, 2) dense_mfma_kernel(DenseParams p) {
   using S = DenseMfma<D, NV>;
