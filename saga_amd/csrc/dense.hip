@@ -494,14 +494,14 @@ __global__ void __launch_bounds__(256, 2) dense_mfma_kernel(DenseParams p) {
       }
     if constexpr (kF16) {
       // what f16 terms in the first unit leave of weights below 2^-16, at most 2^-25: in a unit 2^40 times smaller, and
-      // then in steps of 2^12 (8 terms reach the last bit of the smallest float; a NaN leaves nothing)
+      // then in steps of 2^12 (8 terms reach the last bit of the smallest float)
       float unit = 1.f;
 #pragma unroll 1  // a peeled pass spills
       for (int k = 0; k < 8; ++k) {
-        bool left = false;
+        uint32_t left = 0u;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) left |= x[i] > 0.f || x[i] < 0.f;
-        if (!__any(left)) break;
+        for (int i = 0; i < 8; ++i) left |= __float_as_uint(x[i]);
+        if (!__any((left & 0x7fffffffu) != 0u)) break;
         const float up = k == 0 ? 0x1p40f : 0x1p12f;
         unit *= k == 0 ? 0x1p-40f : 0x1p-12f;
         u32x4 pt;
